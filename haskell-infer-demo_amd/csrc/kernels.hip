@@ -30,6 +30,7 @@
  *                       no K split across blocks); 4 <= M <= 16 inside the FFN entry points,
  *                       which keep the intermediate chunk-major for it, 8 <= M <= 15 on
  *                       row-major rows in gemm_int4_bf16
+ *   rows_gemm_kernel    M > 16: row tiles x tile pairs a block, the rows staged in LDS step by step
  *   mfma_gemm_kernel    2 <= M <= 16 where the above do not fit: v_mfma_f32_16x16x32_bf16, K
  *                       split across blocks
  *   rmsnorm_kernel, residual_add_kernel, silu_mul_packed_kernel: the norm, the residual update
@@ -1339,23 +1340,12 @@ __global__ __launch_bounds__(1024) void gemv_rows16_kernel(
  * contiguous bytes, M / 2 whole cache lines, where the row-major rows give 16 half lines. The
  * A stream is what bounds this kernel (down at M = 16 without its A loads: 6.0 us against
  * 13.1), and the chunk-major order takes it from 13.1 to 8.6-8.7 us.
- *
- * More than 16 row-major rows (gemm_int4_bf16 beyond M = 16): blockIdx.y takes rows
- * 16 y .. 16 y + 15, so the slices run in one launch and their blocks read each weight tile at
- * about the same time (the repeats are served by the caches). */
+ */
 template <bool OUT_F32, int NL, int D, bool CM>
 __global__ __launch_bounds__(1024) void gemv_rows16x_kernel(
     const uint16_t *__restrict__ x, int M, const uint8_t *__restrict__ wt,
     const uint16_t *__restrict__ st, void *__restrict__ out, int N, int K,
     uint16_t *residual) {
-    if (!CM && blockIdx.y > 0) {
-        const int m0 = (int)blockIdx.y * 16;
-        x += (size_t)m0 * K;
-        out = static_cast<char *>(out) + (size_t)m0 * N * (OUT_F32 ? 4 : 2);
-        if (residual) residual += (size_t)m0 * N;
-        M -= m0;
-    }
-    if (M > 16) M = 16;
     constexpr int SK = 16;
     __shared__ f32x4_t red[SK * 64];
     const int G = K >> 7;
@@ -1463,128 +1453,205 @@ __global__ __launch_bounds__(1024) void gemv_rows16x_kernel(
     }
 }
 
-/* Beyond 16 row-major rows (gemm_int4_bf16): gemv_rows16x_kernel's layout (16 waves a block,
- * wave ks taking groups ks + 16 i, A loaded per lane from memory, one LDS meeting at the end),
- * but a wave takes TPW adjacent tile pairs and runs each A operand against all of them, so a
- * block reads its 16 rows of A once for TPW tile pairs: the A bytes the CUs take in (every block
- * reads all of K for its rows) shrink TPW times. blockIdx.y takes rows 16 y .. 16 y + 15. */
-template <bool OUT_F32, int NL, int D, int TPW>
-__global__ __launch_bounds__(1024) void gemv_rows16w_kernel(
-    const uint16_t *__restrict__ x, int M, const uint8_t *__restrict__ wt,
-    const uint16_t *__restrict__ st, void *__restrict__ out, int N, int K) {
-    {
-        const int m0 = (int)blockIdx.y * 16;
-        x += (size_t)m0 * K;
-        out = static_cast<char *>(out) + (size_t)m0 * N * (OUT_F32 ? 4 : 2);
-        M = min(16, M - m0);
+/* Stores one value a lane: row m, row r of `tile`. For the pair, lanes of r < 4 hold gate rows and
+ * the lanes four further the matching up rows, so every lane has to come here. */
+template <int OUT>
+__device__ __forceinline__ void rows_store(float v, bool ok, int m, int tile, int r, int M, int N, void *out,
+                                           uint16_t *residual, int cm) {
+    if (OUT == kOutPairSilu) {
+        /* column r < 4 of a tile has gate row r, column r + 4 the matching up row */
+        const float upv = dpp_f32<kDppRowShl4>(v);
+        if (r < 4 && ok) {
+            const float gate = bf16_widen(bf16_rne(v));
+            const float up = bf16_widen(bf16_rne(upv));
+            reinterpret_cast<uint16_t *>(out)[act_index(m, tile * 4 + r, M, N >> 1, cm)] =
+                silu_mul_bf16(gate, up);
+        }
+    } else if (ok) {
+        const size_t o = (size_t)m * N + tile * 8 + r;
+        if (OUT == kOutF32) {
+            reinterpret_cast<float *>(out)[o] = v;
+        } else {
+            const uint16_t ob = bf16_rne(v);
+            /* plan F2: the residual, already BF16(residual + sublayer), gains the output */
+            if (residual) residual[o] = (uint16_t)(bf16_add2(residual[o], ob) & 0xFFFFu);
+            reinterpret_cast<uint16_t *>(out)[o] = ob;
+        }
     }
-    constexpr int SK = 16;
-    extern __shared__ f32x4_t redw[]; /* [SK][TPW][64 lanes] */
+}
+
+/* More than 16 rows: a block of WN x WK waves owns WN * TPW tile pairs and 16 MT activation rows
+ * over all of K. In each step wave (wn, wk) takes group c WK + wk of its TPW tile pairs from memory
+ * and unpacks it once for all MT row tiles; the block's rows of the WK groups are staged in LDS,
+ * shared by the WN waves of a group and double-buffered (they come through registers: a step's loads are
+ * issued before the step before it is computed and stored to LDS after it). The rows lie as
+ * [group][row][16 chunks], chunk c of a row in slot c ^ (row & 15), so the 16 lanes of one
+ * ds_read_b128 pass hit 16 distinct 16-byte bank slots.
+ * The offset of the unpacked codes (0.75 + code/32) leaves the sums as in gemv_rows_kernel, by
+ * MFMAs against a constant -0.75, but their result is the same for every column: one chain of four
+ * a row tile is the start value of the sums of all TPW tile pairs, so it costs 1 / TPW of theirs.
+ *
+ * What bounds it at 128 rows is the matrix cores with the unpack and the LDS reads close behind
+ * (gate/up 2560 x 19456: 8.9 / 7 / 6.7 us of 26.6 at the 1.9 GHz the card runs there), and the
+ * barrier of each step, which keeps the three from overlapping fully; with staging by waves of
+ * their own and three buffers it was no faster (24.0 against 26.6 us there, 24.8 against 20.5 on
+ * the down projection). Below 32 rows it is the barriers and the latency of a step.
+ * Whole calls, on the 16-row launches before / here: gate/up 2560 x 19456 M = 32 / 64 / 128
+ * 18.5 / 36.9 / 71.5 -> 12.2 / 16.4 / 26.5 us; 5120 x 34816 M = 50 / 128 197 / 482 -> 44 / 84;
+ * down 9728 x 2560 M = 32 / 64 / 128 24.4 / 36.2 / 57.8 -> 12.6 / 15.5 / 20.5. */
+template <int OUT, int MT, int TPW, int WN, int WK>
+__global__ __launch_bounds__(WN * WK * 64) void rows_gemm_kernel(
+    const uint16_t *__restrict__ x, int M, const uint8_t *__restrict__ wt,
+    const uint16_t *__restrict__ st, void *__restrict__ out, int N, int K, int Y, uint16_t *residual) {
+    constexpr int T = WN * WK * 64;
+    constexpr int ROWS = 16 * MT;
+    constexpr int CHUNKS = WK * ROWS * 16; /* 16-byte chunks of one staged step */
+    constexpr int XL = (CHUNKS + T - 1) / T;
+    extern __shared__ uint4 smem4[]; /* two steps; then the wave reduction */
     const int G = K >> 7;
     const int tiles = N >> 3;
-    const int lane = threadIdx.x & 63;
-    const int ks = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int q = lane >> 4;
-    const int n = lane & 15;
-    const int r = n & 7;
-    int tile[TPW];
-#pragma unroll
-    for (int p = 0; p < TPW; ++p) tile[p] = 2 * ((int)blockIdx.x * TPW + p) + (n >> 3);
+    const int NT = (tiles + 1) >> 1;
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wn = wave % WN, wk = wave / WN;
+    /* the Y row slices of one column block run on one XCD (block b on XCD b % 8), next to each
+     * other, so the weight comes from HBM once */
+    const int b8 = (int)blockIdx.x >> 3;
+    const int y = b8 % Y;
+    const int tpb = ((b8 / Y) * 8 + ((int)blockIdx.x & 7)) * WN * TPW;
+    if (tpb >= NT) return;
+    const int tp0 = tpb + wn * TPW;
+    const int m0 = y * ROWS;
+    const int rows = min(M - m0, ROWS);
+    const int q = lane >> 4, n = lane & 15, r = n & 7;
 
-    /* 1. every scale, then every weight piece of this wave (a tile past N reads zeros) */
-    const __amdgpu_buffer_rsrc_t wr = make_rsrc(wt, (uint32_t)((size_t)N * K / 2));
-    const __amdgpu_buffer_rsrc_t sr = make_rsrc(st, (uint32_t)((size_t)N * G * 2));
-    uint4 buf[NL][TPW];
-    uint16_t sbits[NL][TPW];
-#pragma unroll
-    for (int i = 0; i < NL; ++i)
+    /* descriptors: this wave's tiles (a tile past N is past them and reads zeros), the block's rows */
+    const uint32_t tile_bytes = (uint32_t)G * 512;
+    const int wtiles = __builtin_amdgcn_readfirstlane(max(0, min(2 * TPW, tiles - 2 * tp0)));
+    const size_t tile0 = (size_t)(wtiles ? 2 * tp0 : 0);
+    const __amdgpu_buffer_rsrc_t wr = make_rsrc(wt + tile0 * tile_bytes, (uint32_t)wtiles * tile_bytes);
+    const __amdgpu_buffer_rsrc_t sr = make_rsrc(st + tile0 * G * 8, (uint32_t)(wtiles * G) * 16);
+    const __amdgpu_buffer_rsrc_t xr = make_rsrc(x + (size_t)m0 * K, (uint32_t)rows * K * 2);
+
+    uint4 wbuf[TPW];
+    uint16_t sbuf[TPW];
+    auto load_w = [&](int c) { /* this wave's group of step c (past the range: zeros) */
+        const int g = c * WK + wk;
+        const uint32_t past = g < G ? 0u : kOob;
 #pragma unroll
         for (int p = 0; p < TPW; ++p) {
-            const int g = ks + i * SK;
-            const bool ok = tile[p] < tiles && g < G;
-            const uint32_t unit = (uint32_t)(tile[p] * G + g);
-            sbits[i][p] = buf_load_u16(sr, ok ? unit * 16 + (uint32_t)r * 2 : kOob);
+            const uint32_t unit = (uint32_t)((2 * p + (n >> 3)) * G + g);
+            sbuf[p] = buf_load_u16(sr, (unit * 16 + (uint32_t)r * 2) | past);
         }
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int i = 0; i < NL; ++i) {
 #pragma unroll
         for (int p = 0; p < TPW; ++p) {
-            const int g = ks + i * SK;
-            const bool ok = tile[p] < tiles && g < G;
-            const uint32_t unit = (uint32_t)(tile[p] * G + g);
-            buf[i][p] = buf_load16_stream(wr, ok ? unit * 512 + (uint32_t)(q * 8 + r) * 16 : kOob);
+            const uint32_t unit = (uint32_t)((2 * p + (n >> 3)) * G + g);
+            wbuf[p] = buf_load16_stream(wr, (unit * 512 + (uint32_t)(q * 8 + r) * 16) | past);
         }
-        __builtin_amdgcn_sched_barrier(0);
-    }
-
-    /* 2. the A operands of group i: for MFMA t, row n, k = 128 g + 32 t + 8 q .. + 7 */
-    const __amdgpu_buffer_rsrc_t xr = make_rsrc(x, (uint32_t)M * K * 2);
-    const bool row_ok = n < M;
-    const uint32_t row_off = (uint32_t)(n * K + q * 8) * 2;
-    uint4 av[D][4];
-    auto load_a = [&](int i) {
-        const int g = ks + i * SK;
-        const bool ok = row_ok && g < G;
-#pragma unroll
-        for (int t = 0; t < 4; ++t)
-            av[i % D][t] = buf_load16(xr, ok ? row_off + (uint32_t)(g * 128 + 32 * t) * 2 : kOob);
     };
+    /* a thread's chunks of a step: chunk i of [group][row][16 chunks], its slot chunk ^ (row & 15) */
+    uint4 xv[XL];
+    auto load_x = [&](int c) {
 #pragma unroll
-    for (int i = 0; i < D && i < NL; ++i) load_a(i);
+        for (int it = 0; it < XL; ++it) {
+            const int i = it * T + tid;
+            const int row = (i >> 4) % ROWS;
+            const int g = c * WK + i / (ROWS * 16);
+            const bool ok = g < G && row < rows && (CHUNKS % T == 0 || i < CHUNKS);
+            xv[it] = buf_load16(xr, ok ? (uint32_t)(row * K + g * 128 + (i & 15) * 8) * 2 : kOob);
+        }
+    };
+    auto stage_x = [&](int buf) {
+#pragma unroll
+        for (int it = 0; it < XL; ++it) {
+            const int i = it * T + tid;
+            if (CHUNKS % T == 0 || i < CHUNKS)
+                smem4[buf * CHUNKS + (i ^ ((i >> 4) & 15))] = xv[it];
+        }
+    };
 
-    /* 3. per group and tile pair, four product MFMAs and four offset MFMAs, as rows16x */
+    const int steps = (G + WK - 1) / WK;
+    load_x(0);
+    __builtin_amdgcn_sched_barrier(0);
+    load_w(0);
+    __builtin_amdgcn_sched_barrier(0);
+    stage_x(0);
+    __syncthreads();
+
     const uint4 offs = make_uint4(0xBF40BF40u, 0xBF40BF40u, 0xBF40BF40u, 0xBF40BF40u);
-    f32x4_t acc[TPW];
+    f32x4_t acc[MT][TPW];
 #pragma unroll
-    for (int p = 0; p < TPW; ++p) acc[p] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-    for (int i = 0; i < NL; ++i) {
-        if (ks + i * SK < G) { /* wave-uniform */
+        for (int p = 0; p < TPW; ++p) acc[mt][p] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+
+    for (int c0 = 0; c0 < steps; c0 += 2) {
+#pragma unroll
+        for (int v = 0; v < 2; ++v) { /* the buffer of step c */
+            const int c = c0 + v;
+            load_x(c + 1);
+            __builtin_amdgcn_sched_barrier(0);
+            bf16x8_t bv[TPW][4];
+            float sc[TPW];
 #pragma unroll
             for (int p = 0; p < TPW; ++p) {
-                const uint32_t words[4] = {buf[i][p].x, buf[i][p].y, buf[i][p].z, buf[i][p].w};
-                f32x4_t d = {0.0f, 0.0f, 0.0f, 0.0f};
+                const uint32_t words[4] = {wbuf[p].x, wbuf[p].y, wbuf[p].z, wbuf[p].w};
 #pragma unroll
-                for (int t = 0; t < 4; ++t) {
-                    const bf16x8_t a = __builtin_bit_cast(bf16x8_t, av[i % D][t]);
-                    d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, unpack8(words[t]), d, 0, 0, 0);
-                    d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, __builtin_bit_cast(bf16x8_t, offs),
-                                                                d, 0, 0, 0);
-                }
-                const float sc = bf16_widen(sbits[i][p]);
-#pragma unroll
-                for (int j = 0; j < 4; ++j) acc[p][j] = fmaf(sc, d[j], acc[p][j]);
+                for (int t = 0; t < 4; ++t)
+                    bv[p][t] = unpack8(words[t]);
+                sc[p] = bf16_widen(sbuf[p]);
             }
-        } else {
+            load_w(c + 1);
+            if (c < steps) { /* block-uniform */
+                const uint4 *xa = smem4 + (v & 1) * CHUNKS + (wk * ROWS + n) * 16;
 #pragma unroll
-            for (int p = 0; p < TPW; ++p) asm volatile("" ::"v"(buf[i][p].x), "v"(sbits[i][p]));
+                for (int mt = 0; mt < MT; ++mt) {
+                    bf16x8_t a[4];
+#pragma unroll
+                    for (int t = 0; t < 4; ++t)
+                        a[t] = __builtin_bit_cast(bf16x8_t, xa[mt * 256 + ((4 * t + q) ^ n)]);
+                    f32x4_t dx = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                    for (int t = 0; t < 4; ++t)
+                        dx = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[t], __builtin_bit_cast(bf16x8_t, offs),
+                                                                     dx, 0, 0, 0);
+#pragma unroll
+                    for (int p = 0; p < TPW; ++p) {
+                        f32x4_t d = dx;
+#pragma unroll
+                        for (int t = 0; t < 4; ++t)
+                            d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[t], bv[p][t], d, 0, 0, 0);
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) acc[mt][p][j] = fmaf(sc[p], d[j], acc[mt][p][j]);
+                    }
+                }
+            }
+            stage_x((v + 1) & 1);
+            __syncthreads();
         }
-        if (i + D < NL) load_a(i + D);
     }
 
-    /* 4. the 16 waves in LDS, summed in wave order; lane (n, q) holds rows 4 q + j of column n */
+    /* the WK waves of a column group meet in LDS; then the block's waves take D register j of tile t,
+     * a rolled loop (unrolled over tiles and registers this code was several times the main loop) */
+    constexpr int TILES = MT * TPW;
+    f32x4_t *red = reinterpret_cast<f32x4_t *>(smem4); /* [WN][TILES][WK][64 lanes] */
 #pragma unroll
-    for (int p = 0; p < TPW; ++p) redw[(ks * TPW + p) * 64 + lane] = acc[p];
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int p = 0; p < TPW; ++p)
+            red[((wn * TILES + mt * TPW + p) * WK + wk) * 64 + lane] = acc[mt][p];
     __syncthreads();
-    if (ks >= TPW) return;
-    const int p = ks; /* wave p finishes tile pair p */
-    f32x4_t sum = redw[p * 64 + lane];
-    for (int w = 1; w < SK; ++w) {
-        const f32x4_t v = redw[(w * TPW + p) * 64 + lane];
+    for (int i = wave; i < WN * TILES * 4; i += WN * WK) {
+        const int j = i & 3, t = i >> 2;
+        const int mt = (t % TILES) / TPW, tp = tpb + (t / TILES) * TPW + t % TPW;
+        if (tp >= NT || mt * 16 >= rows) continue; /* wave-uniform */
+        float v = 0.0f;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) sum[j] += v[j];
-    }
-    const int tl = 2 * ((int)blockIdx.x * TPW + p) + (n >> 3);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const int m = 4 * q + j;
-        if (m < M && tl < tiles) {
-            const size_t o = (size_t)m * N + tl * 8 + r;
-            const float row_sum = 32.0f * sum[j];
-            if (OUT_F32) reinterpret_cast<float *>(out)[o] = row_sum;
-            else reinterpret_cast<uint16_t *>(out)[o] = bf16_rne(row_sum);
-        }
+        for (int w = 0; w < WK; ++w) v += red[(t * WK + w) * 64 + lane][j];
+        v *= 32.0f; /* the unpacked codes are 1/32 of theirs */
+        const int mr = mt * 16 + 4 * q + j, tile = 2 * tp + (n >> 3);
+        rows_store<OUT>(v, mr < rows && tile < tiles, m0 + mr, tile, r, M, N, out, residual, 0);
     }
 }
 
@@ -2007,7 +2074,7 @@ int launch_rows16x_nl(const uint16_t *x, int M, const uint8_t *w, const uint16_t
                       int N, int K, hipStream_t stream, uint16_t *residual) {
     constexpr int D = NL <= 5 ? NL : NL <= 9 ? 4 : 3;
     const int pairs = (N / 8 + 1) / 2;
-    launch_k((gemv_rows16x_kernel<OUT_F32, NL, D, CM>), dim3(pairs, CM ? 1 : (M + 15) / 16),
+    launch_k((gemv_rows16x_kernel<OUT_F32, NL, D, CM>), dim3(pairs),
              dim3(1024), 0, stream, x, M, w, s, out, N, K, residual);
     return hip_status(hipGetLastError(), "gemv rows16x launch");
 }
@@ -2028,36 +2095,72 @@ int launch_rows16x(const uint16_t *x, int M, const uint8_t *w, const uint16_t *s
     return 1;
 }
 
-/* Beyond 16 row-major rows: gemv_rows16w_kernel with as many tile pairs a wave (4, 2 or 1) as
- * still leaves a block a CU across the 16-row slices. Returns 1 when K is beyond its shapes. */
-template <bool OUT_F32, int NL, int TPW>
-int launch_rows16w_t(const uint16_t *x, int M, const uint8_t *w, const uint16_t *s, void *out,
-                     int N, int K, hipStream_t stream) {
-    constexpr int D = TPW >= 4 ? 1 : 2;
-    const int pairs = (N / 8 + 1) / 2;
-    launch_k((gemv_rows16w_kernel<OUT_F32, NL, D, TPW>), dim3((pairs + TPW - 1) / TPW, (M + 15) / 16),
-             dim3(1024), (size_t)16 * TPW * 64 * sizeof(f32x4_t), stream, x, M, w, s, out, N, K);
-    return hip_status(hipGetLastError(), "gemv rows16w launch");
+template <int OUT, int MT, int TPW, int WN, int WK>
+int launch_rows_gemm_cfg(const uint16_t *x, int M, const uint8_t *w, const uint16_t *s, void *out, int N,
+                         int K, hipStream_t stream, uint16_t *residual) {
+    constexpr size_t stage = (size_t)2 * WK * 16 * MT * 256, reduce = (size_t)WK * WN * MT * TPW * 1024;
+    constexpr size_t smem = stage > reduce ? stage : reduce;
+    static_assert(smem <= kMaxLds, "the two staged steps and the reduction fit a block's LDS");
+    constexpr size_t elem = OUT == kOutF32 ? 4 : 2;
+    const int cols = (((N / 8 + 1) / 2 + WN * TPW - 1) / (WN * TPW) + 7) / 8 * 8;
+    /* a launch of at most 2^21 blocks (a grid holds fewer than 2^32 threads): in practice all rows */
+    const int most = std::max(1, (1 << 21) / cols) * 16 * MT;
+    for (int m0 = 0; m0 < M; m0 += most) {
+        const int rows = std::min(M - m0, most), slices = (rows + 16 * MT - 1) / (16 * MT);
+        const size_t o = (size_t)m0 * (OUT == kOutPairSilu ? N / 2 : N);
+        launch_k((rows_gemm_kernel<OUT, MT, TPW, WN, WK>), dim3((unsigned)cols * slices), dim3(WN * WK * 64),
+                 smem, stream, x + (size_t)m0 * K, rows, w, s, static_cast<char *>(out) + o * elem, N, K,
+                 slices, residual ? residual + o : nullptr);
+        const int st = hip_status(hipGetLastError(), "rows gemm launch");
+        if (st) return st;
+    }
+    return W4A16_OK;
 }
 
-template <bool OUT_F32, int NL>
-int launch_rows16w_nl(const uint16_t *x, int M, const uint8_t *w, const uint16_t *s, void *out,
-                      int N, int K, hipStream_t stream) {
-    const int pairs = (N / 8 + 1) / 2;
-    const int slices = (M + 15) / 16;
-    const int cus = device_cus();
-    if ((pairs / 4) * slices >= cus) return launch_rows16w_t<OUT_F32, NL, 4>(x, M, w, s, out, N, K, stream);
-    if ((pairs / 2) * slices >= cus) return launch_rows16w_t<OUT_F32, NL, 2>(x, M, w, s, out, N, K, stream);
-    return 1;
-}
-
-template <bool OUT_F32>
-int launch_rows16w(const uint16_t *x, int M, const uint8_t *w, const uint16_t *s, void *out, int N,
-                   int K, hipStream_t stream) {
-    const int nl = (K / 128 + 15) / 16;
-    if (nl <= 2) return launch_rows16w_nl<OUT_F32, 2>(x, M, w, s, out, N, K, stream);
-    if (nl <= 3) return launch_rows16w_nl<OUT_F32, 3>(x, M, w, s, out, N, K, stream);
-    return 1;
+/* More than 16 rows: the block shape whose estimated time is least, base + step * steps * rounds,
+ * with steps = ceil(groups / WK) and rounds the blocks of the fullest CU. The two constants of a
+ * shape are a least-squares fit (relative error 5 to 13 %) to its times over 16 weights, K 1024 to
+ * 17408 and N 1024 to 34816, and 17 to 128 rows; the choice is on average within 2 % of the best
+ * shape there. No shape serves all: at 32 rows 9728 x 2560 takes 12.6 us as 1 x 2 x 1 x 8 (row
+ * tiles x tile pairs a wave x column groups x groups a step) and 20 as 2 x 2 x 3 x 4, which takes
+ * 12.4 us where 2560 x 19456 takes 17 as 1 x 2 x 1 x 8. */
+template <int OUT>
+int launch_rows_gemm(const uint16_t *x, int M, const uint8_t *w, const uint16_t *s, void *out, int N,
+                     int K, hipStream_t stream, uint16_t *residual = nullptr) {
+    struct Shape {
+        int rows, tile_pairs, groups; /* a block's rows / 16 and tile pairs, groups a step */
+        float base, step;             /* us */
+    };
+    static constexpr Shape shapes[] = {
+        {1, 2, 8, 2.96f, 1.178f}, {1, 4, 4, 3.60f, 0.642f},  {1, 6, 4, 3.39f, 0.979f},
+        {2, 4, 4, 3.56f, 1.096f}, {2, 6, 4, 4.70f, 1.246f},  {2, 9, 4, 6.10f, 1.598f},
+        {2, 10, 2, 5.27f, 0.994f}, {4, 10, 2, 6.89f, 1.708f}, {2, 6, 2, 4.96f, 0.756f},
+    };
+    const int G = K / 128, tile_pairs = (N / 8 + 1) / 2, cus = device_cus();
+    int best = 0;
+    float least = 0.0f;
+    for (int i = 0; i < (int)(sizeof(shapes) / sizeof(shapes[0])); ++i) {
+        const Shape &c = shapes[i];
+        const long long blocks = (long long)((M + 16 * c.rows - 1) / (16 * c.rows)) *
+                                 ((tile_pairs + c.tile_pairs - 1) / c.tile_pairs);
+        const float t = c.base + c.step * (float)((G + c.groups - 1) / c.groups) *
+                                     (float)((blocks + cus - 1) / cus);
+        if (i == 0 || t < least) {
+            best = i;
+            least = t;
+        }
+    }
+    switch (best) {
+        case 0: return launch_rows_gemm_cfg<OUT, 1, 2, 1, 8>(x, M, w, s, out, N, K, stream, residual);
+        case 1: return launch_rows_gemm_cfg<OUT, 1, 2, 2, 4>(x, M, w, s, out, N, K, stream, residual);
+        case 2: return launch_rows_gemm_cfg<OUT, 1, 3, 2, 4>(x, M, w, s, out, N, K, stream, residual);
+        case 3: return launch_rows_gemm_cfg<OUT, 2, 2, 2, 4>(x, M, w, s, out, N, K, stream, residual);
+        case 4: return launch_rows_gemm_cfg<OUT, 2, 2, 3, 4>(x, M, w, s, out, N, K, stream, residual);
+        case 5: return launch_rows_gemm_cfg<OUT, 2, 3, 3, 4>(x, M, w, s, out, N, K, stream, residual);
+        case 6: return launch_rows_gemm_cfg<OUT, 2, 2, 5, 2>(x, M, w, s, out, N, K, stream, residual);
+        case 7: return launch_rows_gemm_cfg<OUT, 4, 2, 5, 2>(x, M, w, s, out, N, K, stream, residual);
+        default: return launch_rows_gemm_cfg<OUT, 2, 3, 2, 2>(x, M, w, s, out, N, K, stream, residual);
+    }
 }
 
 template <bool PAIR, bool OUT_F32>
@@ -2393,37 +2496,25 @@ int check_gemm_args(const void *a, const void *p, const void *s, const void *o, 
 
 /* Rows of x: M = 1 takes the v_dot2 GEMV; 2 <= M <= 16 the few-row MFMA kernels where their
  * staged rows fit a block's LDS, otherwise the split-K MFMA form, one pass over the weight for
- * all rows; larger M runs on 16-row slices. */
+ * all rows; larger M the row-tiled GEMM. */
 template <int OUT>
 static int run_rows(const uint16_t *x, int M, const uint8_t *w, const uint16_t *s, void *out,
                     int N, int K, hipStream_t stream, int cm = 0) {
     constexpr bool PAIR = OUT == kOutPairSilu;
     constexpr bool F32 = OUT == kOutF32;
-    const int out_cols = PAIR ? N / 2 : N;
-    const size_t out_elem = F32 ? 4 : 2;
-    /* beyond 16 rows (no pair, row-major): all the 16-row slices in one launch of the
-     * registers-fed kernel, and at exactly 16 rows where the LDS-staged kernel cannot hold K */
-    if (!PAIR && !cm && M > 16) {
-        const int st = launch_rows16w<F32>(x, M, w, s, out, N, K, stream);
-        if (st <= 0) return st;
-    }
-    if (!PAIR && !cm && (M > 16 || (M == 16 && rows16_smem(16, K, 16) > kMaxLds))) {
+    if (M > 16) return launch_rows_gemm<OUT>(x, M, w, s, out, N, K, stream);
+    /* at exactly 16 rows where the LDS-staged kernel cannot hold K: the registers-fed kernel */
+    if (!PAIR && !cm && M == 16 && rows16_smem(16, K, 16) > kMaxLds) {
         const int st = launch_rows16x<F32>(x, M, w, s, out, N, K, stream);
         if (st <= 0) return st;
     }
-    for (int m0 = 0; m0 < M; m0 += 16) {
-        const int rows = std::min(16, M - m0);
-        const uint16_t *xs = x + (size_t)m0 * K;
-        void *os = static_cast<char *>(out) + (size_t)m0 * out_cols * out_elem;
-        /* one row: the v_dot2 GEMVs, except a pair operand past the block-staged kernel's K
-         * (then the MFMA form with one live row) */
-        const bool gemv = rows == 1 && (!PAIR || K <= kMaxGemvK);
-        int st = gemv ? launch_gemv<PAIR, F32>(xs, w, s, os, N, K, stream)
-                      : launch_rows<PAIR, F32>(xs, rows, w, s, os, N, K, stream, nullptr, cm);
-        if (st > 0) st = launch_mfma<OUT>(xs, rows, w, s, os, N, K, stream, nullptr, cm);
-        if (st) return st;
-    }
-    return W4A16_OK;
+    /* one row: the v_dot2 GEMVs, except a pair operand past the block-staged kernel's K
+     * (then the MFMA form with one live row) */
+    const bool gemv = M == 1 && (!PAIR || K <= kMaxGemvK);
+    int st = gemv ? launch_gemv<PAIR, F32>(x, w, s, out, N, K, stream)
+                  : launch_rows<PAIR, F32>(x, M, w, s, out, N, K, stream, nullptr, cm);
+    if (st > 0) st = launch_mfma<OUT>(x, M, w, s, out, N, K, stream, nullptr, cm);
+    return st;
 }
 
 extern "C" int gemm_int4_bf16(const uint16_t *a, const uint8_t *packed, const uint16_t *scales,
@@ -2721,6 +2812,7 @@ extern "C" int mlp_int4_residual_norm_bf16(uint16_t *residual, const uint16_t *s
         if (st > 0) st = launch_mfma<kOutBf16>(act, M, dnp, dns, out, hidden, inter, s, residual);
         return st;
     }
+    if (M > 16) return launch_rows_gemm<kOutBf16>(act, M, dnp, dns, out, hidden, inter, s, residual);
     st = run_rows<kOutBf16>(act, M, dnp, dns, out, hidden, inter, s);
     if (st) return st;
     const long long chunks = (long long)M * hidden / 8;

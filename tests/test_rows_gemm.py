@@ -1,0 +1,73 @@
+"""More than 16 activation rows: the row-tiled GEMM (rows_gemm_kernel) through each of its block
+shapes, at the edges of their row tiles, tile pairs and K steps, against the oracle. The
+tolerances are the suite's (assert_parity): 2 BF16 ULP and rel-L2 1e-3 of the double-accumulated
+product."""
+
+import numpy as np
+import pytest
+import torch
+
+import w4a16
+from conftest import assert_parity
+from oracle import oracle
+from test_gpu_parity import from_dev, make_ffn, make_weight, norm_inputs, to_dev
+
+pytestmark = pytest.mark.gpu
+
+# (rows, N, K): one half-filled tile pair of one group; then every block shape (row tiles x tile
+# pairs x groups a step) where the launcher's estimate picks it, with odd tile counts, rows that do
+# not fill the row tiles and K that does not fill the steps
+SHAPES = [
+    (17, 8, 128),
+    (33, 2568, 1664),    # 1 x 2 x 8
+    (33, 9736, 640),     # 1 x 4 x 4
+    (17, 9736, 640),     # 1 x 6 x 4
+    (17, 12296, 128),    # 2 x 4 x 4
+    (50, 12296, 640),    # 2 x 6 x 4
+    (33, 16424, 1920),   # 2 x 9 x 4
+    (63, 19464, 640),    # 2 x 10 x 2
+    (127, 34824, 640),   # 4 x 10 x 2
+    (120, 24584, 768),   # 2 x 6 x 2
+]
+
+
+@pytest.mark.parametrize("m,n,k", SHAPES)
+def test_linear_parity(cuda, m, n, k):
+    print(f"gemm M={m} N={n} K={k}", flush=True)
+    p, s = make_weight(n, k, seed=n + k)
+    x = oracle.synth_activation(m, k, seed=m + n)
+    w = w4a16.TiledWeight.from_artifact(p, s, n, k, device=cuda)
+    out = from_dev(w4a16.gemm_int4_bf16(to_dev(x, cuda), w))
+    assert_parity(out, oracle.gemm_bf16(x, p, s, n, k), f"gemm M={m} N={n} K={k}")
+
+
+@pytest.mark.parametrize("m,hidden,inter", [(17, 128, 128), (65, 640, 9728), (129, 640, 2176)])
+def test_ffn_forms(cuda, m, hidden, inter):
+    """The gate/up pair and the down projection, each stage against the oracle on its own inputs
+    (end to end a BF16 rounding of the intermediate that falls the other way moves an output by
+    up to 2^-8 |act| |w|, which is no error of either stage); then the forms around them, which
+    run the same kernels and have to agree bit for bit: the FP32 partial rounds to the BF16
+    output, and plan F2 is the MLP of the normed sum, with the residual gaining exactly it."""
+    print(f"ffn M={m} H={hidden} I={inter}", flush=True)
+    gup, gus, dp, ds = make_ffn(hidden, inter, layer=40)
+    gu = w4a16.TiledWeight.from_artifact(gup, gus, 2 * inter, hidden, pair=True, device=cuda)
+    dn = w4a16.TiledWeight.from_artifact(dp, ds, hidden, inter, device=cuda)
+    x = oracle.synth_activation(m, hidden, seed=9)
+    xd = to_dev(x, cuda)
+    act = w4a16.gate_up_silu(xd, gu)
+    mid = oracle.gemm_bf16(x, gup, gus, 2 * inter, hidden)
+    assert_parity(from_dev(act), oracle.silu_mul_packed(mid, m, inter), f"gate/up M={m} I={inter}")
+    down = w4a16.gemm_int4_bf16(act, dn)
+    assert_parity(from_dev(down), oracle.gemm_bf16(from_dev(act), dp, ds, hidden, inter), f"down M={m} K={inter}")
+    assert torch.equal(w4a16.mlp_int4(xd, gu, dn), down)
+    f32 = w4a16.mlp_int4(xd, gu, dn, partial_f32=True)
+    assert torch.equal(f32.to(torch.bfloat16).view(torch.int16), down.view(torch.int16))
+
+    res, nw = norm_inputs(m, hidden, 1, seed=10)
+    sub = oracle.synth_activation(m, hidden, seed=11)
+    summed, _ = oracle.residual_norm_bf16(res, sub, nw, 1, 1e-6)
+    resd = to_dev(res, cuda)
+    got = w4a16.mlp_int4_residual_norm(resd, to_dev(sub, cuda), to_dev(nw, cuda), 1, 1e-6, gu, dn)
+    normed = w4a16.rmsnorm(to_dev(summed, cuda), to_dev(nw, cuda), 1, 1e-6)
+    assert torch.equal(got, w4a16.mlp_int4(normed, gu, dn))
+    assert np.array_equal(from_dev(resd), oracle.residual_add_bf16(summed, from_dev(got)))
