@@ -30,6 +30,8 @@
  *                       no K split across blocks); 4 <= M <= 16 inside the FFN entry points,
  *                       which keep the intermediate chunk-major for it, 8 <= M <= 15 on
  *                       row-major rows in gemm_int4_bf16
+ *   rows_stream_kernel  up to 16 rows, long K or many tile pairs a CU: one block a CU, its rows and
+ *                       K range staged in LDS once, its units dealt evenly to its waves
  *   rows_gemm_kernel    M > 16: row tiles x tile pairs a block, the rows staged in LDS step by step
  *   mfma_gemm_kernel    2 <= M <= 16 where the above do not fit: v_mfma_f32_16x16x32_bf16, K
  *                       split across blocks
@@ -1655,6 +1657,183 @@ __global__ __launch_bounds__(WN * WK * 64) void rows_gemm_kernel(
     }
 }
 
+/* Up to 16 rows, a long K or many tile pairs a CU: one block of 16 waves a CU owns TPB <= 16 tile
+ * pairs and GS groups of K, and stages its rows of those groups in LDS once (up to 160 KB; chunk c
+ * of row m in slot c ^ m, or, with CM, as the chunk-major activation lies in memory). The block's
+ * TPB x GS units (a group of a tile pair, 1 KiB of weight) are then dealt to its waves in equal
+ * contiguous ranges, tile pair by tile pair, so no wave idles where TPB is no multiple of
+ * anything; a range of at most GS units touches at most two tile pairs, whose sums stay in two
+ * accumulators and meet in LDS at the end. No barrier stands between the staging and the end, and
+ * each wave keeps PD units in flight. With S > 1 the S blocks of a tile pair meet through mailbox
+ * slots (see slot_put), which hold the rows < M only.
+ *
+ * It takes the place of the split-K MFMA form where the few-row kernels' rows do not fit LDS or
+ * leave one or two blocks a CU, and of gemv_rows16x_kernel where its one-tile-pair blocks of 16
+ * waves need a second round. What bounds it is the VALU (52 instructions a unit: unpack 28, MFMA
+ * 8, scale 5, addresses) next to the stream itself, after 2 to 3 us of staging; by block stamps
+ * at M = 16, K = 5120, 9 tile pairs a CU: staged at 3-5 us, waves done at 11-20, end at 21.
+ * PD = 2 measured as fast as 3 and faster than 4 to 8 (the weight loads of the first units stand
+ * ahead of other waves' staging loads in the CU's memory queue). Before / here: gate/up
+ * 5120 x 34816 M = 8 / 12 / 16 37.6 / 64.8 / 65.4 -> 23.5 / 26 / 25 us; down 17408 x 5120 (chunk-
+ * major) M = 4 / 8 / 16 22.8 / 23.5 / 27.4 -> 15.5 / 16.5 / 18.9. */
+template <int OUT, bool CM, bool SPLIT>
+__global__ __launch_bounds__(1024) void rows_stream_kernel(
+    const uint16_t *__restrict__ x, int M, const uint8_t *__restrict__ wt,
+    const uint16_t *__restrict__ st, void *__restrict__ out, int N, int K, int TPB, int S, int GS,
+    uint64_t *__restrict__ partial, unsigned *__restrict__ counters, uint16_t *residual, int cm) {
+    constexpr int W = 16, PD = 2;
+    extern __shared__ uint4 smem4[];
+    const int G = K >> 7;
+    const int tiles = N >> 3;
+    const int NT = (tiles + 1) >> 1;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int cb = (int)blockIdx.x / S, ks = (int)blockIdx.x % S;
+    const int g0 = ks * GS;
+    const int gs = min(G - g0, GS);
+    const int tpb0 = cb * TPB;
+    const int ntp = min(TPB, NT - tpb0);
+    const int q = lane >> 4, n = lane & 15, r = n & 7;
+
+    /* 1. the block's rows and K range into LDS */
+    const __amdgpu_buffer_rsrc_t xr = make_rsrc(x, (uint32_t)M * K * 2);
+    const int nlds = gs * M * 16;
+    const uint32_t mdiv = div_magic(M);
+    for (int j = wave; j * 64 < nlds; j += W) {
+        const int pos = j * 64 + lane;
+        uint32_t off;
+        if (CM) {
+            off = (uint32_t)(g0 * M * 256 + pos * 16); /* as it lies in memory */
+        } else {
+            const int gl = div_small(pos >> 4, mdiv);
+            const int m = (pos >> 4) - gl * M;
+            off = (uint32_t)(m * K + (g0 + gl) * 128 + ((pos & 15) ^ (m & 15)) * 8) * 2;
+        }
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(
+            xr, (__attribute__((address_space(3))) void *)(smem4 + j * 64), 16, pos < nlds ? off : kOob, 0, 0, 0);
+    }
+
+    /* 2. this wave's units */
+    const int U = ntp * gs;
+    const int u0 = U * wave / W, u1 = U * (wave + 1) / W;
+    const int p0 = __builtin_amdgcn_readfirstlane(u0 / gs);
+    const uint32_t tile_bytes = (uint32_t)G * 512;
+    const int btiles = min(2 * ntp, tiles - 2 * tpb0);
+    const __amdgpu_buffer_rsrc_t wr = make_rsrc(wt + (size_t)(2 * tpb0) * tile_bytes, (uint32_t)btiles * tile_bytes);
+    const __amdgpu_buffer_rsrc_t sr = make_rsrc(st + (size_t)(2 * tpb0) * G * 8, (uint32_t)(btiles * G) * 16);
+    const uint32_t lane_w = (uint32_t)(n >> 3) * tile_bytes + (uint32_t)(q * 8 + r) * 16;
+    const uint32_t lane_s = (uint32_t)((n >> 3) * G * 16 + r * 2);
+    uint4 wbuf[PD];
+    uint16_t sbuf[PD];
+    int lu = u0, lp = p0, lg = u0 - p0 * gs; /* the next unit to load */
+    auto load_w = [&](int b) {
+        const uint32_t past = lu < u1 ? 0u : kOob;
+        const uint32_t unit = (uint32_t)(2 * lp * G + g0 + lg);
+        sbuf[b] = buf_load_u16(sr, (lane_s + unit * 16) | past);
+        wbuf[b] = buf_load16_stream(wr, (lane_w + unit * 512) | past);
+        ++lu;
+        if (++lg == gs) {
+            lg = 0;
+            ++lp;
+        }
+    };
+#pragma unroll
+    for (int b = 0; b < PD; ++b) {
+        load_w(b);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    __builtin_amdgcn_s_waitcnt(vm_enc(2 * PD));
+    __syncthreads();
+
+    const uint4 offs = make_uint4(0xBF40BF40u, 0xBF40BF40u, 0xBF40BF40u, 0xBF40BF40u);
+    f32x4_t acc = {0.0f, 0.0f, 0.0f, 0.0f}, first = acc;
+    const int arow = min(n, M - 1);
+    int cu = u0, cg = u0 - p0 * gs;
+    const int cnt = u1 - u0;
+    for (int i0 = 0; i0 < cnt; i0 += PD) {
+#pragma unroll
+        for (int b = 0; b < PD; ++b) {
+            if (cu < u1) { /* wave-uniform */
+                const float sc = bf16_widen(sbuf[b]);
+                const uint32_t words[4] = {wbuf[b].x, wbuf[b].y, wbuf[b].z, wbuf[b].w};
+                const uint4 *xa = smem4 + cg * M * 16;
+                f32x4_t d = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                for (int t = 0; t < 4; ++t) {
+                    const bf16x8_t a = __builtin_bit_cast(
+                        bf16x8_t, CM ? xa[(4 * t + q) * M + arow] : xa[arow * 16 + ((4 * t + q) ^ (arow & 15))]);
+                    d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, unpack8(words[t]), d, 0, 0, 0);
+                    d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, __builtin_bit_cast(bf16x8_t, offs), d, 0, 0, 0);
+                }
+#pragma unroll
+                for (int j = 0; j < 4; ++j) acc[j] = fmaf(sc, d[j], acc[j]);
+                ++cu;
+                if (++cg == gs) { /* the end of a tile pair: the wave's range may go on into the next */
+                    cg = 0;
+                    if (cu < u1) {
+                        first = acc;
+                        acc = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+                    }
+                }
+            }
+            load_w(b);
+        }
+    }
+    __syncthreads();
+    f32x4_t *red = reinterpret_cast<f32x4_t *>(smem4); /* [16 waves][its first, its second pair][64 lanes] */
+    const bool two = cnt > 0 && (u1 - 1) / gs != p0;
+    red[(wave * 2 + 0) * 64 + lane] = two ? first : acc;
+    red[(wave * 2 + 1) * 64 + lane] = acc;
+    __syncthreads();
+    /* a wave finishes whole tile pairs; the partials of pair p lie with the waves whose range
+     * [U w / 16, U (w + 1) / 16) meets its units [p gs, (p + 1) gs), and are added in wave order */
+    for (int p = wave; p < ntp; p += W) {
+        const int tp = tpb0 + p;
+        const int tile = 2 * tp + (n >> 3);
+        f32x4_t sum = {0.0f, 0.0f, 0.0f, 0.0f};
+        for (int w = p * W / ntp; w < W && U * w / W < (p + 1) * gs; ++w) {
+            if (U * (w + 1) / W <= p * gs) continue;
+            const int second = U * w / W < p * gs ? 1 : 0;
+            const f32x4_t v = red[(w * 2 + second) * 64 + lane];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) sum[j] += v[j];
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) sum[j] *= 32.0f; /* the unpacked codes are 1/32 of theirs */
+        if (SPLIT) {
+            const size_t stride = (size_t)NT * 16 * M; /* slots of one split */
+            uint64_t *slot = partial + (size_t)tp * 16 * M + 4 * q * 16 + n; /* row 4 q + j: 16 j on */
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                if (4 * q + j < M) slot_put(slot + ks * stride + j * 16, sum[j]);
+            if (split_arrive(&counters[tp], lane) != (unsigned)(S - 1)) continue;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) sum[j] = 0.0f;
+            for (int k0 = 0; k0 < S; k0 += 4) { /* sixteen round trips to the coherence point at once */
+                uint64_t v[4][4];
+#pragma unroll
+                for (int k = 0; k < 4; ++k)
+#pragma unroll
+                    for (int j = 0; j < 4; ++j)
+                        v[k][j] = k0 + k < S && 4 * q + j < M ? slot_peek(slot + (k0 + k) * stride + j * 16) : 0ull;
+#pragma unroll
+                for (int k = 0; k < 4; ++k)
+#pragma unroll
+                    for (int j = 0; j < 4; ++j)
+                        if (k0 + k < S && 4 * q + j < M)
+                            sum[j] += slot_take(slot + (k0 + k) * stride + j * 16, v[k][j]);
+            }
+            if (lane == 0)
+                __hip_atomic_store(&counters[tp], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int m = 4 * q + j;
+            rows_store<OUT>(sum[j], m < M && tile < tiles, m, tile, r, M, N, out, residual, cm);
+        }
+    }
+}
+
 /* RMSNorm of each row (one block a row): BF16(x * rsqrt(sum x^2 / cols + eps) * (bias + w)),
  * FP32 arithmetic (reference csrc/kernels/flashinfer_norm.cu:22-76). Each thread holds CH
  * 8-value chunks of the row, all loaded before any use, so a row costs one load round trip;
@@ -2179,20 +2358,53 @@ int launch_rows16(const uint16_t *x, int M, const uint8_t *w, const uint16_t *s,
     return 1;
 }
 
+template <int OUT, bool CM>
+int launch_rows_stream(const uint16_t *x, int M, const uint8_t *w, const uint16_t *s, void *out, int N,
+                       int K, hipStream_t stream, uint16_t *residual, int cm);
+
 template <bool PAIR, bool OUT_F32>
 int launch_rows(const uint16_t *x, int M, const uint8_t *w, const uint16_t *s, void *out, int N,
                 int K, hipStream_t stream, uint16_t *residual = nullptr, int cm = 0) {
-    /* long K (the staged rows would not fit LDS): registers-fed A from M = 8 (9 with the
-     * residual epilogue) to 15; at 16 the split-K MFMA form is faster. C1 down, medians of
-     * interleaved whole-call runs, split-K or LDS-staged against rows16x: M = 8 20.5 / 19.9 us,
-     * 10 22.7 / 21.0, 13 23.9 / 22.6, 14 24.2 / 23.4, 15 24.2 / 23.9, 16 24.4 / 24.6; at M = 8
-     * plan F2 23.3 against 23.6, and M = 4 and 6 tie. */
-    if (!PAIR && M >= (residual ? 9 : 8) && M <= 15 && rows16_smem(M, K, 16) > kMaxLds)
-        return launch_rows16x<OUT_F32>(x, M, w, s, out, N, K, stream, residual);
-    if (M > 8 && M <= 16 && !residual)
-        return launch_rows16<PAIR, OUT_F32>(x, M, w, s, out, N, K, stream, cm);
-    if (M < 2 || M > 8) return 1;
+    constexpr int OUT = PAIR ? kOutPairSilu : OUT_F32 ? kOutF32 : kOutBf16;
+    if (M < 2 || M > 16) return 1;
     const int pairs = (K / 128 + 1) / 2;
+    const int tile_pairs = (N / 8 + 1) / 2;
+    /* A block a CU over its whole share (rows_stream_kernel) where the few-row kernels' blocks are
+     * few and large. The pair, M <= 8: their staged rows leave two blocks a CU or fewer and a CU has
+     * four tile pairs or more (5120 x 17408 M = 4 / 6 / 8 14.7 / 17.6 / 23.1 against 15.1 / 15.5 /
+     * 15.9 us; 3200 x 17152 M = 6 / 8 11.4 / 13.4 against 11.3 / 11.5; with three tile pairs a CU,
+     * 3584 x 12288 M = 8, 10.0 against 10.4). Otherwise (a long K): more than one tile pair a CU
+     * (17408 x 5120 M = 2 / 3 / 8 19.5 / 20.7 / 32.5 against 15.6 / 15.8 / 17.0), from a K that
+     * falls with the rows (10240 x 5120 M = 2 / 3 / 4 8.7 / 11.8 / 13.6 against 11.6 / 11.7 / 11.8,
+     * 8704 x 5120 M = 4 / 6 10.9 / 12.9 against 10.9 / 11.2). */
+    const int long_pairs = M == 2 ? 48 : M == 3 ? 40 : M == 4 ? 34 : 20;
+    const bool stream_few = PAIR ? rows_smem(M, K, 0) > kMaxLds / 3 && tile_pairs >= 4 * device_cus()
+                                 : pairs > long_pairs && tile_pairs > device_cus();
+    if (M <= 8 && stream_few) {
+        const int st = launch_rows_stream<OUT, false>(x, M, w, s, out, N, K, stream, residual, cm);
+        if (st <= 0) return st;
+    }
+    /* A long K whose staged 9 to 16 rows would not fit LDS: the same kernel at more than one tile
+     * pair a CU, as in launch_down_cm (so the FFN's down projection and this one, row-major, sum in
+     * the same order), and at 16 rows (9728 x 2560 13.2 us registers-fed, 10.0 here; 14336 x 3584
+     * 19.9 against 13.6); registers-fed otherwise, and from M = 8 without the residual epilogue (C1
+     * down, whole calls: 20.5 us LDS-staged, 19.9 registers-fed; with the residual 23.3 / 23.6). */
+    const bool long_k = !PAIR && rows16_smem(M, K, 16) > kMaxLds;
+    if (M >= 9 && long_k && (M == 16 || tile_pairs > device_cus())) {
+        const int st = launch_rows_stream<OUT, false>(x, M, w, s, out, N, K, stream, residual, cm);
+        if (st <= 0) return st;
+    }
+    if (M >= (residual ? 9 : 8) && long_k) {
+        const int st = launch_rows16x<OUT_F32>(x, M, w, s, out, N, K, stream, residual);
+        if (st <= 0) return st;
+    }
+    if (M > 8 && !residual) {
+        const int st = launch_rows16<PAIR, OUT_F32>(x, M, w, s, out, N, K, stream, cm);
+        if (st <= 0) return st;
+    }
+    /* 9 to 16 rows that the LDS-staged tile-pair form cannot hold: M = 9 / 16 5120 x 34816 62 / 65 us
+     * in the split-K MFMA form, 25 / 25 here; 4096 x 24576 34 / 37 against 17 / 18 */
+    if (M > 8) return launch_rows_stream<OUT, false>(x, M, w, s, out, N, K, stream, residual, cm);
     /* two rows on the matrix-core GEMV: the gate/up pair at 7 to 12 group pairs (four waves of
      * three) and the long K of the C1 down projection, 37 to 48 pairs (sixteen of three). Whole
      * C1 FFN call at M = 2: 12.58-12.66 us against 13.70-13.99 on this kernel's few-row form
@@ -2338,6 +2550,91 @@ MfmaPlan plan_mfma(int M, int N, int K) {
     p.partial_bytes = p.S > 1 ? (size_t)p.S * NT * 16 * M * sizeof(uint64_t) : 0;
     p.ncounters = p.S > 1 ? (size_t)NT : 0;
     return p;
+}
+
+/* The plan of rows_stream_kernel: the K split S (GS groups each) and the tile pairs a block that
+ * take the least estimated time in one round of blocks, one a CU: 0.033 us a unit, 16 ns a KiB of
+ * staged rows, 2.2 us for the combine of a split (fitted to M = 2..16 on 17 weights). S is at most
+ * what the split-K MFMA form would use, so the scratch reserved for that serves here too. */
+struct StreamPlan {
+    int S, GS, TPB, grid;
+    size_t smem, partial_bytes, ncounters;
+};
+
+bool plan_stream(int M, int N, int K, bool split, StreamPlan *plan) {
+    const int G = K / 128, NT = (N / 8 + 1) / 2, cus = device_cus();
+    float least = 0.0f;
+    for (int s = 1; s <= (split ? std::min(8, (G + kGMax - 1) / kGMax) : 1); ++s) {
+        StreamPlan p{};
+        p.GS = (G + s - 1) / s;
+        p.S = (G + p.GS - 1) / p.GS;
+        p.TPB = (int)(((long long)NT * p.S + cus - 1) / cus);
+        p.grid = (NT + p.TPB - 1) / p.TPB * p.S;
+        p.smem = std::max(((size_t)p.GS * M * 256 + 1023) / 1024 * 1024, (size_t)32 * 1024);
+        if (p.smem > kMaxLds || p.TPB > 16) continue;
+        const float t = 0.033f * p.TPB * p.GS + 0.004f * p.GS * M + (p.S > 1 ? 2.2f : 0.0f);
+        if (least == 0.0f || t < least) {
+            least = t;
+            p.partial_bytes = p.S > 1 ? (size_t)p.S * NT * 16 * M * sizeof(uint64_t) : 0;
+            p.ncounters = p.S > 1 ? (size_t)NT : 0;
+            *plan = p;
+        }
+    }
+    return least > 0.0f;
+}
+
+/* Whether split_scratch can serve this size without allocating. */
+bool split_scratch_ready(size_t partial_bytes, size_t ncounters) {
+    if (t_fixed.active) return partial_bytes <= t_fixed.partial_bytes && ncounters <= t_fixed.ncounters;
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return false;
+    std::lock_guard<std::mutex> lock(g_scratch_mu);
+    return partial_bytes <= g_scratch[dev].partial_bytes && ncounters <= g_scratch[dev].ncounters;
+}
+
+/* Returns 1 when no plan fits, or when it would have to grow the scratch under graph capture (the
+ * kernels it stands in for need none, so a first call that was captured before stays possible). */
+template <int OUT, bool CM>
+int launch_rows_stream(const uint16_t *x, int M, const uint8_t *w, const uint16_t *s, void *out, int N,
+                       int K, hipStream_t stream, uint16_t *residual, int cm) {
+    constexpr bool PAIR = OUT == kOutPairSilu;
+    StreamPlan p{};
+    if (!plan_stream(M, N, K, !PAIR, &p)) return 1;
+    uint64_t *partial = nullptr;
+    unsigned *counters = nullptr;
+    if (p.S > 1) {
+        if (!split_scratch_ready(p.partial_bytes, p.ncounters)) {
+            hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+            const int st = hip_status(hipStreamIsCapturing(stream, &cap), "hipStreamIsCapturing");
+            if (st) return st;
+            if (cap != hipStreamCaptureStatusNone || t_fixed.active) return 1;
+        }
+        const int st = split_scratch(p.partial_bytes, p.ncounters, &partial, &counters);
+        if (st) return st;
+    }
+    if (!PAIR && p.S > 1)
+        launch_k((rows_stream_kernel<OUT, CM, !PAIR>), dim3(p.grid), dim3(1024), p.smem, stream, x, M, w, s,
+                 out, N, K, p.TPB, p.S, p.GS, partial, counters, residual, cm);
+    else
+        launch_k((rows_stream_kernel<OUT, CM, false>), dim3(p.grid), dim3(1024), p.smem, stream, x, M, w, s,
+                 out, N, K, p.TPB, 1, p.GS, partial, counters, residual, cm);
+    return hip_status(hipGetLastError(), "rows stream launch");
+}
+
+/* The down projection of M rows of a chunk-major activation (64 to 192 groups of K). Up to one
+ * tile pair a CU the registers-fed kernel; beyond, its blocks of a tile pair and 16 waves take a
+ * second round, and one block a CU over its whole share is faster (M = 4 / 16: 8704 x 5120 12.7 / 14.4
+ * against 10.6 / 12.0 us, 13824 x 5120 19.5 / 22.3 against 13.8 / 16.1; 9728 x 2560, 160 tile pairs,
+ * 7.3 / 8.2 against 8.5 / 9.5; 12288 x 4096, 256, 9.7 / 11.4 against 10.5 / 13.4). */
+template <bool OUT_F32>
+int launch_down_cm(const uint16_t *act, int M, const uint8_t *w, const uint16_t *s, void *out, int N, int K,
+                   hipStream_t stream, uint16_t *residual = nullptr) {
+    if ((N / 8 + 1) / 2 > device_cus()) {
+        const int st = launch_rows_stream<OUT_F32 ? kOutF32 : kOutBf16, true>(act, M, w, s, out, N, K, stream,
+                                                                             residual, 0);
+        if (st <= 0) return st;
+    }
+    return launch_rows16x<OUT_F32, true>(act, M, w, s, out, N, K, stream, residual);
 }
 
 /* ---- The allocation-free scratch ------------------------------------------------------------
@@ -2494,20 +2791,14 @@ int check_gemm_args(const void *a, const void *p, const void *s, const void *o, 
 /* C ABI                                                                                     */
 /* ---------------------------------------------------------------------------------------- */
 
-/* Rows of x: M = 1 takes the v_dot2 GEMV; 2 <= M <= 16 the few-row MFMA kernels where their
- * staged rows fit a block's LDS, otherwise the split-K MFMA form, one pass over the weight for
- * all rows; larger M the row-tiled GEMM. */
+/* Rows of x: M = 1 takes the v_dot2 GEMV; 2 <= M <= 16 the kernels of launch_rows, or the split-K
+ * MFMA form where they have no shape; larger M the row-tiled GEMM. */
 template <int OUT>
 static int run_rows(const uint16_t *x, int M, const uint8_t *w, const uint16_t *s, void *out,
                     int N, int K, hipStream_t stream, int cm = 0) {
     constexpr bool PAIR = OUT == kOutPairSilu;
     constexpr bool F32 = OUT == kOutF32;
     if (M > 16) return launch_rows_gemm<OUT>(x, M, w, s, out, N, K, stream);
-    /* at exactly 16 rows where the LDS-staged kernel cannot hold K: the registers-fed kernel */
-    if (!PAIR && !cm && M == 16 && rows16_smem(16, K, 16) > kMaxLds) {
-        const int st = launch_rows16x<F32>(x, M, w, s, out, N, K, stream);
-        if (st <= 0) return st;
-    }
     /* one row: the v_dot2 GEMVs, except a pair operand past the block-staged kernel's K
      * (then the MFMA form with one live row) */
     const bool gemv = M == 1 && (!PAIR || K <= kMaxGemvK);
@@ -2564,8 +2855,8 @@ static int mlp_common(const uint16_t *normed, const uint8_t *gup, const uint16_t
         if (st < 0) return st;
         st = run_rows<kOutPairSilu>(normed, M, gup, gus, act, 2 * inter, hidden, s, 1);
         if (st) return st;
-        return out_f32 ? launch_rows16x<true, true>(act, M, dnp, dns, out, hidden, inter, s)
-                       : launch_rows16x<false, true>(act, M, dnp, dns, out, hidden, inter, s);
+        return out_f32 ? launch_down_cm<true>(act, M, dnp, dns, out, hidden, inter, s)
+                       : launch_down_cm<false>(act, M, dnp, dns, out, hidden, inter, s);
     }
     st = gate_up_silu_int4_bf16(normed, gup, gus, act, M, hidden, inter, stream);
     if (st) return st;
@@ -2720,8 +3011,8 @@ static int mlp_norm_common(const uint16_t *residual, const uint16_t *norm_w, int
     }
     if (st) return st;
     if (cm)
-        return out_f32 ? launch_rows16x<true, true>(act, M, dnp, dns, out, hidden, inter, s)
-                       : launch_rows16x<false, true>(act, M, dnp, dns, out, hidden, inter, s);
+        return out_f32 ? launch_down_cm<true>(act, M, dnp, dns, out, hidden, inter, s)
+                       : launch_down_cm<false>(act, M, dnp, dns, out, hidden, inter, s);
     return out_f32 ? run_rows<kOutF32>(act, M, dnp, dns, out, hidden, inter, s)
                    : run_rows<kOutBf16>(act, M, dnp, dns, out, hidden, inter, s);
 }
@@ -2801,7 +3092,7 @@ extern "C" int mlp_int4_residual_norm_bf16(uint16_t *residual, const uint16_t *s
     st = launch_rmsnorm(normed, residual, norm_w, hidden, M, na.bias, eps, s, sublayer);
     if (!st) st = run_rows<kOutPairSilu>(normed, M, gup, gus, act, 2 * inter, hidden, s, cm);
     if (st) return st;
-    if (cm) return launch_rows16x<false, true>(act, M, dnp, dns, out, hidden, inter, s, residual);
+    if (cm) return launch_down_cm<false>(act, M, dnp, dns, out, hidden, inter, s, residual);
     if (M == 1 && dn_pairs > kMaxLoads) {
         /* the down kernel adds the output into the (already updated) residual itself */
         st = launch_xwave<false>(act, dnp, dns, out, hidden, inter, s, residual, nullptr);
