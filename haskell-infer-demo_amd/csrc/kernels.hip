@@ -30,9 +30,10 @@
  *                       no K split across blocks); 4 <= M <= 16 inside the FFN entry points,
  *                       which keep the intermediate chunk-major for it, 8 <= M <= 15 on
  *                       row-major rows in gemm_int4_bf16
- *   rows_stream_kernel  up to 16 rows, long K or many tile pairs a CU: one block a CU, its rows and
- *                       K range staged in LDS once, its units dealt evenly to its waves
- *   rows_gemm_kernel    M > 16: row tiles x tile pairs a block, the rows staged in LDS step by step
+ *   rows_stream_kernel  the down projection of up to 16 rows, more than one tile pair a CU: one
+ *                       block a CU, its rows staged in LDS once, its units dealt evenly to its waves
+ *   rows_gemm_kernel    M > 16, and up to 16 rows where the above give a CU too few blocks: row tiles
+ *                       x tile pairs a block, the rows staged in LDS step by step
  *   mfma_gemm_kernel    2 <= M <= 16 where the above do not fit: v_mfma_f32_16x16x32_bf16, K
  *                       split across blocks
  *   rmsnorm_kernel, residual_add_kernel, silu_mul_packed_kernel: the norm, the residual update
@@ -1482,29 +1483,34 @@ __device__ __forceinline__ void rows_store(float v, bool ok, int m, int tile, in
     }
 }
 
-/* More than 16 rows: a block of WN x WK waves owns WN * TPW tile pairs and 16 MT activation rows
+/* Rows by tiles of 16: a block of WN x WK waves owns WN * TPW tile pairs and 16 MT activation rows
  * over all of K. In each step wave (wn, wk) takes group c WK + wk of its TPW tile pairs from memory
  * and unpacks it once for all MT row tiles; the block's rows of the WK groups are staged in LDS,
- * shared by the WN waves of a group and double-buffered (they come through registers: a step's loads are
- * issued before the step before it is computed and stored to LDS after it). The rows lie as
- * [group][row][16 chunks], chunk c of a row in slot c ^ (row & 15), so the 16 lanes of one
- * ds_read_b128 pass hit 16 distinct 16-byte bank slots.
- * The offset of the unpacked codes (0.75 + code/32) leaves the sums as in gemv_rows_kernel, by
- * MFMAs against a constant -0.75, but their result is the same for every column: one chain of four
- * a row tile is the start value of the sums of all TPW tile pairs, so it costs 1 / TPW of theirs.
+ * shared by the WN waves of a group and double-buffered (they come through registers: a step's
+ * loads are issued before the step before it is computed and stored to LDS after it). The rows lie
+ * as [group][row][16 chunks], chunk c of a row in slot c ^ (row & 15), so the 16 lanes of one
+ * ds_read_b128 pass hit 16 distinct 16-byte bank slots. With CM the activation is chunk-major.
+ * The offset of the unpacked codes (0.75 + code/32) leaves the sums as in gemv_rows_kernel, by an
+ * MFMA against a constant -0.75 after that of the codes. One chain of offsets for all TPW tile
+ * pairs would save up to half of the MFMAs (128 rows of 2560 x 19456 26.5 us instead of 28.9), but
+ * its sums reach five times the result before they cancel: 1.3 times as many outputs then round
+ * other than the exact product's (3.3e-4 of them against 2.5e-4 here and 2.6e-4 in gemv_rows16_kernel).
  *
  * What bounds it at 128 rows is the matrix cores with the unpack and the LDS reads close behind
- * (gate/up 2560 x 19456: 8.9 / 7 / 6.7 us of 26.6 at the 1.9 GHz the card runs there), and the
+ * (gate/up 2560 x 19456: 12.8 / 7 / 6.7 us of 28.9 at the 1.9 GHz the card runs there), and the
  * barrier of each step, which keeps the three from overlapping fully; with staging by waves of
- * their own and three buffers it was no faster (24.0 against 26.6 us there, 24.8 against 20.5 on
- * the down projection). Below 32 rows it is the barriers and the latency of a step.
- * Whole calls, on the 16-row launches before / here: gate/up 2560 x 19456 M = 32 / 64 / 128
- * 18.5 / 36.9 / 71.5 -> 12.2 / 16.4 / 26.5 us; 5120 x 34816 M = 50 / 128 197 / 482 -> 44 / 84;
- * down 9728 x 2560 M = 32 / 64 / 128 24.4 / 36.2 / 57.8 -> 12.6 / 15.5 / 20.5. */
-template <int OUT, int MT, int TPW, int WN, int WK>
+ * their own and three buffers it was no faster there and slower on the down projection (24.8
+ * against 20.5). With few rows it is the barriers and the latency of a step: at 16 rows of 5120 x
+ * 34816 the weight stream alone in this block shape takes 19 of 23 us.
+ * Whole calls, on the kernels before / here: gate/up 2560 x 19456 M = 32 / 64 / 128 18.1 / 35.3 / 68.9 ->
+ * 12.8 / 18.0 / 28.9 us; 5120 x 34816 M = 16 / 32 / 64 / 128 61 / 120 / 241 / 480 -> 23.5 / 29.7 / 49 / 97;
+ * down 9728 x 2560 M = 32 / 64 / 128 24.2 / 35.9 / 57.4 -> 12.5 / 14.3 / 22.3; 17408 x 5120 M = 16 /
+ * 32 / 64 / 128 24.8 / 61 / 100 / 194 -> 20.6 / 23.7 / 34.9 / 50.2. */
+template <int OUT, int MT, int TPW, int WN, int WK, bool CM>
 __global__ __launch_bounds__(WN * WK * 64) void rows_gemm_kernel(
     const uint16_t *__restrict__ x, int M, const uint8_t *__restrict__ wt,
-    const uint16_t *__restrict__ st, void *__restrict__ out, int N, int K, int Y, uint16_t *residual) {
+    const uint16_t *__restrict__ st, void *__restrict__ out, int N, int K, int Y, uint16_t *residual, int cm) {
+    static_assert(!CM || MT == 1, "a chunk-major activation has at most 16 rows");
     constexpr int T = WN * WK * 64;
     constexpr int ROWS = 16 * MT;
     constexpr int CHUNKS = WK * ROWS * 16; /* 16-byte chunks of one staged step */
@@ -1552,24 +1558,27 @@ __global__ __launch_bounds__(WN * WK * 64) void rows_gemm_kernel(
             wbuf[p] = buf_load16_stream(wr, (unit * 512 + (uint32_t)(q * 8 + r) * 16) | past);
         }
     };
-    /* a thread's chunks of a step: chunk i of [group][row][16 chunks], its slot chunk ^ (row & 15) */
+    /* A thread's chunks of a step, i = (group, row, chunk), the chunk in slot chunk ^ (row & 15); of
+     * a chunk-major activation i = (group, chunk, row), the order in which it lies in memory. */
     uint4 xv[XL];
     auto load_x = [&](int c) {
 #pragma unroll
         for (int it = 0; it < XL; ++it) {
             const int i = it * T + tid;
-            const int row = (i >> 4) % ROWS;
+            const int row = CM ? i & 15 : (i >> 4) % ROWS;
             const int g = c * WK + i / (ROWS * 16);
             const bool ok = g < G && row < rows && (CHUNKS % T == 0 || i < CHUNKS);
-            xv[it] = buf_load16(xr, ok ? (uint32_t)(row * K + g * 128 + (i & 15) * 8) * 2 : kOob);
+            const uint32_t off = CM ? (uint32_t)((g * 16 + ((i >> 4) & 15)) * M + row) * 16
+                                    : (uint32_t)(row * K + g * 128 + (i & 15) * 8) * 2;
+            xv[it] = buf_load16(xr, ok ? off : kOob);
         }
     };
     auto stage_x = [&](int buf) {
 #pragma unroll
         for (int it = 0; it < XL; ++it) {
             const int i = it * T + tid;
-            if (CHUNKS % T == 0 || i < CHUNKS)
-                smem4[buf * CHUNKS + (i ^ ((i >> 4) & 15))] = xv[it];
+            const int slot = CM ? (i & ~255) | (i & 15) << 4 | (((i >> 4) ^ i) & 15) : i ^ ((i >> 4) & 15);
+            if (CHUNKS % T == 0 || i < CHUNKS) smem4[buf * CHUNKS + slot] = xv[it];
         }
     };
 
@@ -1613,17 +1622,15 @@ __global__ __launch_bounds__(WN * WK * 64) void rows_gemm_kernel(
 #pragma unroll
                     for (int t = 0; t < 4; ++t)
                         a[t] = __builtin_bit_cast(bf16x8_t, xa[mt * 256 + ((4 * t + q) ^ n)]);
-                    f32x4_t dx = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-                    for (int t = 0; t < 4; ++t)
-                        dx = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[t], __builtin_bit_cast(bf16x8_t, offs),
-                                                                     dx, 0, 0, 0);
 #pragma unroll
                     for (int p = 0; p < TPW; ++p) {
-                        f32x4_t d = dx;
+                        f32x4_t d = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-                        for (int t = 0; t < 4; ++t)
+                        for (int t = 0; t < 4; ++t) {
                             d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[t], bv[p][t], d, 0, 0, 0);
+                            d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[t], __builtin_bit_cast(bf16x8_t, offs),
+                                                                        d, 0, 0, 0);
+                        }
 #pragma unroll
                         for (int j = 0; j < 4; ++j) acc[mt][p][j] = fmaf(sc[p], d[j], acc[mt][p][j]);
                     }
@@ -1653,34 +1660,30 @@ __global__ __launch_bounds__(WN * WK * 64) void rows_gemm_kernel(
         for (int w = 0; w < WK; ++w) v += red[(t * WK + w) * 64 + lane][j];
         v *= 32.0f; /* the unpacked codes are 1/32 of theirs */
         const int mr = mt * 16 + 4 * q + j, tile = 2 * tp + (n >> 3);
-        rows_store<OUT>(v, mr < rows && tile < tiles, m0 + mr, tile, r, M, N, out, residual, 0);
+        rows_store<OUT>(v, mr < rows && tile < tiles, m0 + mr, tile, r, M, N, out, residual, cm);
     }
 }
 
-/* Up to 16 rows, a long K or many tile pairs a CU: one block of 16 waves a CU owns TPB <= 16 tile
- * pairs and GS groups of K, and stages its rows of those groups in LDS once (up to 160 KB; chunk c
- * of row m in slot c ^ m, or, with CM, as the chunk-major activation lies in memory). The block's
- * TPB x GS units (a group of a tile pair, 1 KiB of weight) are then dealt to its waves in equal
- * contiguous ranges, tile pair by tile pair, so no wave idles where TPB is no multiple of
- * anything; a range of at most GS units touches at most two tile pairs, whose sums stay in two
+/* The down projection of a few rows (K x rows up to 160 KB of LDS) with more than one tile pair a
+ * CU: one block of 16 waves a CU owns TPB <= 16 tile pairs over all of K and stages its rows in LDS
+ * once (chunk c of row m in slot c ^ m or, with CM, as the chunk-major activation lies in memory).
+ * The block's TPB x G units (a group of a tile pair, 1 KiB of weight) are then dealt to its waves in
+ * equal contiguous ranges, tile pair by tile pair, so no wave idles where TPB is no multiple of
+ * anything; a range of at most G units touches at most two tile pairs, whose sums stay in two
  * accumulators and meet in LDS at the end. No barrier stands between the staging and the end, and
- * each wave keeps PD units in flight. With S > 1 the S blocks of a tile pair meet through mailbox
- * slots (see slot_put), which hold the rows < M only.
+ * each wave keeps PD units in flight.
  *
- * It takes the place of the split-K MFMA form where the few-row kernels' rows do not fit LDS or
- * leave one or two blocks a CU, and of gemv_rows16x_kernel where its one-tile-pair blocks of 16
- * waves need a second round. What bounds it is the VALU (52 instructions a unit: unpack 28, MFMA
- * 8, scale 5, addresses) next to the stream itself, after 2 to 3 us of staging; by block stamps
- * at M = 16, K = 5120, 9 tile pairs a CU: staged at 3-5 us, waves done at 11-20, end at 21.
- * PD = 2 measured as fast as 3 and faster than 4 to 8 (the weight loads of the first units stand
- * ahead of other waves' staging loads in the CU's memory queue). Before / here: gate/up
- * 5120 x 34816 M = 8 / 12 / 16 37.6 / 64.8 / 65.4 -> 23.5 / 26 / 25 us; down 17408 x 5120 (chunk-
- * major) M = 4 / 8 / 16 22.8 / 23.5 / 27.4 -> 15.5 / 16.5 / 18.9. */
-template <int OUT, bool CM, bool SPLIT>
+ * What bounds it is the VALU (52 instructions a unit: unpack 28, MFMA 8, scale 5, addresses) next
+ * to the stream itself, after 2 us of staging. PD = 2 measured as fast as 3 and faster than 4 to 8
+ * (the weight loads of the first units stand ahead of other waves' staging loads in the CU's memory
+ * queue). K split across blocks, which would spread few tile pairs better, lost: alternating with
+ * the gate/up kernel the combine's mailbox costs up to 10 us (10240 x 5120 M = 4 22.8 us with three
+ * splits, 11.0 with none). Down projections between gate/up calls, before / here: 17408 x 5120 M = 4
+ * 20.6 -> 14.9 us; 10240 x 5120 M = 4 / 8 12.5 / 12.7 -> 10.4 / 11.1; 8704 x 5120 M = 8 11.3 -> 10.0. */
+template <bool OUT_F32, bool CM>
 __global__ __launch_bounds__(1024) void rows_stream_kernel(
     const uint16_t *__restrict__ x, int M, const uint8_t *__restrict__ wt,
-    const uint16_t *__restrict__ st, void *__restrict__ out, int N, int K, int TPB, int S, int GS,
-    uint64_t *__restrict__ partial, unsigned *__restrict__ counters, uint16_t *residual, int cm) {
+    const uint16_t *__restrict__ st, void *__restrict__ out, int N, int K, int TPB, uint16_t *residual) {
     constexpr int W = 16, PD = 2;
     extern __shared__ uint4 smem4[];
     const int G = K >> 7;
@@ -1688,35 +1691,32 @@ __global__ __launch_bounds__(1024) void rows_stream_kernel(
     const int NT = (tiles + 1) >> 1;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int cb = (int)blockIdx.x / S, ks = (int)blockIdx.x % S;
-    const int g0 = ks * GS;
-    const int gs = min(G - g0, GS);
-    const int tpb0 = cb * TPB;
+    const int tpb0 = (int)blockIdx.x * TPB;
     const int ntp = min(TPB, NT - tpb0);
     const int q = lane >> 4, n = lane & 15, r = n & 7;
 
-    /* 1. the block's rows and K range into LDS */
+    /* 1. the rows into LDS */
     const __amdgpu_buffer_rsrc_t xr = make_rsrc(x, (uint32_t)M * K * 2);
-    const int nlds = gs * M * 16;
+    const int nlds = G * M * 16;
     const uint32_t mdiv = div_magic(M);
     for (int j = wave; j * 64 < nlds; j += W) {
         const int pos = j * 64 + lane;
         uint32_t off;
         if (CM) {
-            off = (uint32_t)(g0 * M * 256 + pos * 16); /* as it lies in memory */
+            off = (uint32_t)pos * 16; /* as it lies in memory */
         } else {
             const int gl = div_small(pos >> 4, mdiv);
             const int m = (pos >> 4) - gl * M;
-            off = (uint32_t)(m * K + (g0 + gl) * 128 + ((pos & 15) ^ (m & 15)) * 8) * 2;
+            off = (uint32_t)(m * K + gl * 128 + ((pos & 15) ^ (m & 15)) * 8) * 2;
         }
         __builtin_amdgcn_raw_ptr_buffer_load_lds(
             xr, (__attribute__((address_space(3))) void *)(smem4 + j * 64), 16, pos < nlds ? off : kOob, 0, 0, 0);
     }
 
     /* 2. this wave's units */
-    const int U = ntp * gs;
+    const int U = ntp * G;
     const int u0 = U * wave / W, u1 = U * (wave + 1) / W;
-    const int p0 = __builtin_amdgcn_readfirstlane(u0 / gs);
+    const int p0 = __builtin_amdgcn_readfirstlane(u0 / G);
     const uint32_t tile_bytes = (uint32_t)G * 512;
     const int btiles = min(2 * ntp, tiles - 2 * tpb0);
     const __amdgpu_buffer_rsrc_t wr = make_rsrc(wt + (size_t)(2 * tpb0) * tile_bytes, (uint32_t)btiles * tile_bytes);
@@ -1725,14 +1725,14 @@ __global__ __launch_bounds__(1024) void rows_stream_kernel(
     const uint32_t lane_s = (uint32_t)((n >> 3) * G * 16 + r * 2);
     uint4 wbuf[PD];
     uint16_t sbuf[PD];
-    int lu = u0, lp = p0, lg = u0 - p0 * gs; /* the next unit to load */
+    int lu = u0, lp = p0, lg = u0 - p0 * G; /* the next unit to load */
     auto load_w = [&](int b) {
         const uint32_t past = lu < u1 ? 0u : kOob;
-        const uint32_t unit = (uint32_t)(2 * lp * G + g0 + lg);
+        const uint32_t unit = (uint32_t)(2 * lp * G + lg);
         sbuf[b] = buf_load_u16(sr, (lane_s + unit * 16) | past);
         wbuf[b] = buf_load16_stream(wr, (lane_w + unit * 512) | past);
         ++lu;
-        if (++lg == gs) {
+        if (++lg == G) {
             lg = 0;
             ++lp;
         }
@@ -1748,7 +1748,7 @@ __global__ __launch_bounds__(1024) void rows_stream_kernel(
     const uint4 offs = make_uint4(0xBF40BF40u, 0xBF40BF40u, 0xBF40BF40u, 0xBF40BF40u);
     f32x4_t acc = {0.0f, 0.0f, 0.0f, 0.0f}, first = acc;
     const int arow = min(n, M - 1);
-    int cu = u0, cg = u0 - p0 * gs;
+    int cu = u0, cg = u0 - p0 * G;
     const int cnt = u1 - u0;
     for (int i0 = 0; i0 < cnt; i0 += PD) {
 #pragma unroll
@@ -1768,7 +1768,7 @@ __global__ __launch_bounds__(1024) void rows_stream_kernel(
 #pragma unroll
                 for (int j = 0; j < 4; ++j) acc[j] = fmaf(sc, d[j], acc[j]);
                 ++cu;
-                if (++cg == gs) { /* the end of a tile pair: the wave's range may go on into the next */
+                if (++cg == G) { /* the end of a tile pair: the wave's range may go on into the next */
                     cg = 0;
                     if (cu < u1) {
                         first = acc;
@@ -1781,55 +1781,30 @@ __global__ __launch_bounds__(1024) void rows_stream_kernel(
     }
     __syncthreads();
     f32x4_t *red = reinterpret_cast<f32x4_t *>(smem4); /* [16 waves][its first, its second pair][64 lanes] */
-    const bool two = cnt > 0 && (u1 - 1) / gs != p0;
+    const bool two = cnt > 0 && (u1 - 1) / G != p0;
     red[(wave * 2 + 0) * 64 + lane] = two ? first : acc;
     red[(wave * 2 + 1) * 64 + lane] = acc;
     __syncthreads();
     /* a wave finishes whole tile pairs; the partials of pair p lie with the waves whose range
-     * [U w / 16, U (w + 1) / 16) meets its units [p gs, (p + 1) gs), and are added in wave order */
+     * [U w / 16, U (w + 1) / 16) meets its units [p G, (p + 1) G), and are added in wave order */
     for (int p = wave; p < ntp; p += W) {
         const int tp = tpb0 + p;
         const int tile = 2 * tp + (n >> 3);
         f32x4_t sum = {0.0f, 0.0f, 0.0f, 0.0f};
-        for (int w = p * W / ntp; w < W && U * w / W < (p + 1) * gs; ++w) {
-            if (U * (w + 1) / W <= p * gs) continue;
-            const int second = U * w / W < p * gs ? 1 : 0;
+        for (int w = p * W / ntp; w < W && U * w / W < (p + 1) * G; ++w) {
+            if (U * (w + 1) / W <= p * G) continue;
+            const int second = U * w / W < p * G ? 1 : 0;
             const f32x4_t v = red[(w * 2 + second) * 64 + lane];
 #pragma unroll
             for (int j = 0; j < 4; ++j) sum[j] += v[j];
         }
 #pragma unroll
         for (int j = 0; j < 4; ++j) sum[j] *= 32.0f; /* the unpacked codes are 1/32 of theirs */
-        if (SPLIT) {
-            const size_t stride = (size_t)NT * 16 * M; /* slots of one split */
-            uint64_t *slot = partial + (size_t)tp * 16 * M + 4 * q * 16 + n; /* row 4 q + j: 16 j on */
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-                if (4 * q + j < M) slot_put(slot + ks * stride + j * 16, sum[j]);
-            if (split_arrive(&counters[tp], lane) != (unsigned)(S - 1)) continue;
-#pragma unroll
-            for (int j = 0; j < 4; ++j) sum[j] = 0.0f;
-            for (int k0 = 0; k0 < S; k0 += 4) { /* sixteen round trips to the coherence point at once */
-                uint64_t v[4][4];
-#pragma unroll
-                for (int k = 0; k < 4; ++k)
-#pragma unroll
-                    for (int j = 0; j < 4; ++j)
-                        v[k][j] = k0 + k < S && 4 * q + j < M ? slot_peek(slot + (k0 + k) * stride + j * 16) : 0ull;
-#pragma unroll
-                for (int k = 0; k < 4; ++k)
-#pragma unroll
-                    for (int j = 0; j < 4; ++j)
-                        if (k0 + k < S && 4 * q + j < M)
-                            sum[j] += slot_take(slot + (k0 + k) * stride + j * 16, v[k][j]);
-            }
-            if (lane == 0)
-                __hip_atomic_store(&counters[tp], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             const int m = 4 * q + j;
-            rows_store<OUT>(sum[j], m < M && tile < tiles, m, tile, r, M, N, out, residual, cm);
+            rows_store<OUT_F32 ? kOutF32 : kOutBf16>(sum[j], m < M && tile < tiles, m, tile, r, M, N, out,
+                                                     residual, 0);
         }
     }
 }
@@ -2274,9 +2249,9 @@ int launch_rows16x(const uint16_t *x, int M, const uint8_t *w, const uint16_t *s
     return 1;
 }
 
-template <int OUT, int MT, int TPW, int WN, int WK>
+template <int OUT, int MT, int TPW, int WN, int WK, bool CM = false>
 int launch_rows_gemm_cfg(const uint16_t *x, int M, const uint8_t *w, const uint16_t *s, void *out, int N,
-                         int K, hipStream_t stream, uint16_t *residual) {
+                         int K, hipStream_t stream, uint16_t *residual, int cm) {
     constexpr size_t stage = (size_t)2 * WK * 16 * MT * 256, reduce = (size_t)WK * WN * MT * TPW * 1024;
     constexpr size_t smem = stage > reduce ? stage : reduce;
     static_assert(smem <= kMaxLds, "the two staged steps and the reduction fit a block's LDS");
@@ -2287,58 +2262,65 @@ int launch_rows_gemm_cfg(const uint16_t *x, int M, const uint8_t *w, const uint1
     for (int m0 = 0; m0 < M; m0 += most) {
         const int rows = std::min(M - m0, most), slices = (rows + 16 * MT - 1) / (16 * MT);
         const size_t o = (size_t)m0 * (OUT == kOutPairSilu ? N / 2 : N);
-        launch_k((rows_gemm_kernel<OUT, MT, TPW, WN, WK>), dim3((unsigned)cols * slices), dim3(WN * WK * 64),
-                 smem, stream, x + (size_t)m0 * K, rows, w, s, static_cast<char *>(out) + o * elem, N, K,
-                 slices, residual ? residual + o : nullptr);
+        launch_k((rows_gemm_kernel<OUT, MT, TPW, WN, WK, CM>), dim3((unsigned)cols * slices),
+                 dim3(WN * WK * 64), smem, stream, x + (size_t)m0 * K, rows, w, s,
+                 static_cast<char *>(out) + o * elem, N, K, slices, residual ? residual + o : nullptr, cm);
         const int st = hip_status(hipGetLastError(), "rows gemm launch");
         if (st) return st;
     }
     return W4A16_OK;
 }
 
-/* More than 16 rows: the block shape whose estimated time is least, base + step * steps * rounds,
- * with steps = ceil(groups / WK) and rounds the blocks of the fullest CU. The two constants of a
- * shape are a least-squares fit (relative error 5 to 13 %) to its times over 16 weights, K 1024 to
- * 17408 and N 1024 to 34816, and 17 to 128 rows; the choice is on average within 2 % of the best
- * shape there. No shape serves all: at 32 rows 9728 x 2560 takes 12.6 us as 1 x 2 x 1 x 8 (row
- * tiles x tile pairs a wave x column groups x groups a step) and 20 as 2 x 2 x 3 x 4, which takes
- * 12.4 us where 2560 x 19456 takes 17 as 1 x 2 x 1 x 8. */
+/* rows_gemm_kernel in the block shape whose estimated time is least: base + steps * (first + more *
+ * (rounds - 1)), with steps = ceil(groups / WK) and rounds the blocks of the fullest CU, counted on
+ * the fullest XCD (column blocks go round the eight XCDs, a column block's row slices stay on one).
+ * A shape's three constants are a least-squares fit (relative error 3 to 8 %) to its times over 22
+ * weights, K 1024 to 17408 and N 1024 to 34816, and 16 to 128 rows; the choice is on average within
+ * 1 % of the best shape there and never more than 20 % off. No shape serves all: at 32 rows
+ * 9728 x 2560 takes 12.0 us as 1 x 2 x 8 (row tiles x tile pairs x groups a step) and 20 as 2 x 6 x
+ * 4, which takes 12.1 us where 2560 x 19456 takes 17 as 1 x 2 x 8. */
 template <int OUT>
 int launch_rows_gemm(const uint16_t *x, int M, const uint8_t *w, const uint16_t *s, void *out, int N,
-                     int K, hipStream_t stream, uint16_t *residual = nullptr) {
+                     int K, hipStream_t stream, uint16_t *residual = nullptr, int cm = 0) {
     struct Shape {
         int rows, tile_pairs, groups; /* a block's rows / 16 and tile pairs, groups a step */
-        float base, step;             /* us */
+        float base, first, more;      /* us */
     };
     static constexpr Shape shapes[] = {
-        {1, 2, 8, 2.96f, 1.178f}, {1, 4, 4, 3.60f, 0.642f},  {1, 6, 4, 3.39f, 0.979f},
-        {2, 4, 4, 3.56f, 1.096f}, {2, 6, 4, 4.70f, 1.246f},  {2, 9, 4, 6.10f, 1.598f},
-        {2, 10, 2, 5.27f, 0.994f}, {4, 10, 2, 6.89f, 1.708f}, {2, 6, 2, 4.96f, 0.756f},
+        {1, 1, 16, 6.02f, 0.60f, 2.11f}, {1, 2, 8, 4.05f, 0.77f, 1.33f},  {1, 3, 8, 4.40f, 0.89f, 1.55f},
+        {1, 4, 4, 3.62f, 0.63f, 0.65f},  {1, 6, 4, 4.13f, 0.80f, 1.18f},  {1, 8, 4, 4.18f, 0.98f, 1.42f},
+        {1, 10, 2, 4.13f, 0.65f, 0.85f}, {2, 4, 4, 4.13f, 0.94f, 1.34f},  {2, 6, 4, 5.07f, 1.09f, 1.77f},
+        {2, 9, 4, 6.50f, 1.45f, 2.33f},  {2, 10, 2, 5.46f, 0.94f, 1.31f}, {2, 6, 2, 4.85f, 0.74f, 0.64f},
+        {4, 10, 2, 6.89f, 1.67f, 2.32f},
     };
-    const int G = K / 128, tile_pairs = (N / 8 + 1) / 2, cus = device_cus();
+    const int G = K / 128, tile_pairs = (N / 8 + 1) / 2, xcd_cus = std::max(1, device_cus() / 8);
     int best = 0;
     float least = 0.0f;
     for (int i = 0; i < (int)(sizeof(shapes) / sizeof(shapes[0])); ++i) {
         const Shape &c = shapes[i];
-        const long long blocks = (long long)((M + 16 * c.rows - 1) / (16 * c.rows)) *
-                                 ((tile_pairs + c.tile_pairs - 1) / c.tile_pairs);
-        const float t = c.base + c.step * (float)((G + c.groups - 1) / c.groups) *
-                                     (float)((blocks + cus - 1) / cus);
+        const long long blocks = ((long long)(tile_pairs + c.tile_pairs - 1) / c.tile_pairs + 7) / 8 *
+                                 ((M + 16 * c.rows - 1) / (16 * c.rows));
+        const float rounds = (float)((blocks + xcd_cus - 1) / xcd_cus);
+        const float t = c.base + (float)((G + c.groups - 1) / c.groups) * (c.first + c.more * (rounds - 1.0f));
         if (i == 0 || t < least) {
             best = i;
             least = t;
         }
     }
     switch (best) {
-        case 0: return launch_rows_gemm_cfg<OUT, 1, 2, 1, 8>(x, M, w, s, out, N, K, stream, residual);
-        case 1: return launch_rows_gemm_cfg<OUT, 1, 2, 2, 4>(x, M, w, s, out, N, K, stream, residual);
-        case 2: return launch_rows_gemm_cfg<OUT, 1, 3, 2, 4>(x, M, w, s, out, N, K, stream, residual);
-        case 3: return launch_rows_gemm_cfg<OUT, 2, 2, 2, 4>(x, M, w, s, out, N, K, stream, residual);
-        case 4: return launch_rows_gemm_cfg<OUT, 2, 2, 3, 4>(x, M, w, s, out, N, K, stream, residual);
-        case 5: return launch_rows_gemm_cfg<OUT, 2, 3, 3, 4>(x, M, w, s, out, N, K, stream, residual);
-        case 6: return launch_rows_gemm_cfg<OUT, 2, 2, 5, 2>(x, M, w, s, out, N, K, stream, residual);
-        case 7: return launch_rows_gemm_cfg<OUT, 4, 2, 5, 2>(x, M, w, s, out, N, K, stream, residual);
-        default: return launch_rows_gemm_cfg<OUT, 2, 3, 2, 2>(x, M, w, s, out, N, K, stream, residual);
+        case 0: return launch_rows_gemm_cfg<OUT, 1, 1, 1, 16>(x, M, w, s, out, N, K, stream, residual, cm);
+        case 1: return launch_rows_gemm_cfg<OUT, 1, 2, 1, 8>(x, M, w, s, out, N, K, stream, residual, cm);
+        case 2: return launch_rows_gemm_cfg<OUT, 1, 3, 1, 8>(x, M, w, s, out, N, K, stream, residual, cm);
+        case 3: return launch_rows_gemm_cfg<OUT, 1, 2, 2, 4>(x, M, w, s, out, N, K, stream, residual, cm);
+        case 4: return launch_rows_gemm_cfg<OUT, 1, 3, 2, 4>(x, M, w, s, out, N, K, stream, residual, cm);
+        case 5: return launch_rows_gemm_cfg<OUT, 1, 4, 2, 4>(x, M, w, s, out, N, K, stream, residual, cm);
+        case 6: return launch_rows_gemm_cfg<OUT, 1, 2, 5, 2>(x, M, w, s, out, N, K, stream, residual, cm);
+        case 7: return launch_rows_gemm_cfg<OUT, 2, 2, 2, 4>(x, M, w, s, out, N, K, stream, residual, cm);
+        case 8: return launch_rows_gemm_cfg<OUT, 2, 2, 3, 4>(x, M, w, s, out, N, K, stream, residual, cm);
+        case 9: return launch_rows_gemm_cfg<OUT, 2, 3, 3, 4>(x, M, w, s, out, N, K, stream, residual, cm);
+        case 10: return launch_rows_gemm_cfg<OUT, 2, 2, 5, 2>(x, M, w, s, out, N, K, stream, residual, cm);
+        case 11: return launch_rows_gemm_cfg<OUT, 2, 3, 2, 2>(x, M, w, s, out, N, K, stream, residual, cm);
+        default: return launch_rows_gemm_cfg<OUT, 4, 2, 5, 2>(x, M, w, s, out, N, K, stream, residual, cm);
     }
 }
 
@@ -2358,9 +2340,36 @@ int launch_rows16(const uint16_t *x, int M, const uint8_t *w, const uint16_t *s,
     return 1;
 }
 
-template <int OUT, bool CM>
+/* rows_stream_kernel; returns 1 when the rows or a CU's tile pairs are past it. */
+template <bool OUT_F32, bool CM>
 int launch_rows_stream(const uint16_t *x, int M, const uint8_t *w, const uint16_t *s, void *out, int N,
-                       int K, hipStream_t stream, uint16_t *residual, int cm);
+                       int K, hipStream_t stream, uint16_t *residual) {
+    const int tile_pairs = (N / 8 + 1) / 2, cus = device_cus();
+    const int TPB = (tile_pairs + cus - 1) / cus;
+    /* the rows, then in their place two partial sums a wave */
+    const size_t smem = std::max(((size_t)(K / 128) * M * 256 + 1023) / 1024 * 1024, (size_t)32 * 1024);
+    if (M > 16 || TPB > 16 || smem > kMaxLds) return 1;
+    launch_k((rows_stream_kernel<OUT_F32, CM>), dim3((tile_pairs + TPB - 1) / TPB), dim3(1024), smem, stream,
+             x, M, w, s, out, N, K, TPB, residual);
+    return hip_status(hipGetLastError(), "rows stream launch");
+}
+
+/* The down projection of M rows of a chunk-major activation (64 to 192 groups of K). Up to one
+ * tile pair a CU the registers-fed kernel; beyond, its blocks of a tile pair and 16 waves take a
+ * second round, and one block a CU over its whole share is faster, or, where the rows do not fit
+ * LDS, the row-tiled GEMM (between gate/up calls, registers-fed against here: 8704 x 5120 M = 8 / 16
+ * 11.3 / 14.0 us, 10.0 / 12.4; 17408 x 5120 M = 4 / 8 / 16 20.6 / 20.6 / 23.7, 14.9 / 19.0 / 20.1;
+ * up to one tile pair a CU 9728 x 2560 M = 4 / 16 7.3 / 7.7 against 8.3 / 10.7). */
+template <bool OUT_F32>
+int launch_down_cm(const uint16_t *act, int M, const uint8_t *w, const uint16_t *s, void *out, int N, int K,
+                   hipStream_t stream, uint16_t *residual = nullptr) {
+    if ((N / 8 + 1) / 2 <= device_cus())
+        return launch_rows16x<OUT_F32, true>(act, M, w, s, out, N, K, stream, residual);
+    const int st = launch_rows_stream<OUT_F32, true>(act, M, w, s, out, N, K, stream, residual);
+    if (st <= 0) return st;
+    return launch_rows_gemm_cfg<OUT_F32 ? kOutF32 : kOutBf16, 1, 2, 1, 8, true>(act, M, w, s, out, N, K, stream,
+                                                                               residual, 0);
+}
 
 template <bool PAIR, bool OUT_F32>
 int launch_rows(const uint16_t *x, int M, const uint8_t *w, const uint16_t *s, void *out, int N,
@@ -2369,42 +2378,42 @@ int launch_rows(const uint16_t *x, int M, const uint8_t *w, const uint16_t *s, v
     if (M < 2 || M > 16) return 1;
     const int pairs = (K / 128 + 1) / 2;
     const int tile_pairs = (N / 8 + 1) / 2;
-    /* A block a CU over its whole share (rows_stream_kernel) where the few-row kernels' blocks are
-     * few and large. The pair, M <= 8: their staged rows leave two blocks a CU or fewer and a CU has
-     * four tile pairs or more (5120 x 17408 M = 4 / 6 / 8 14.7 / 17.6 / 23.1 against 15.1 / 15.5 /
-     * 15.9 us; 3200 x 17152 M = 6 / 8 11.4 / 13.4 against 11.3 / 11.5; with three tile pairs a CU,
-     * 3584 x 12288 M = 8, 10.0 against 10.4). Otherwise (a long K): more than one tile pair a CU
-     * (17408 x 5120 M = 2 / 3 / 8 19.5 / 20.7 / 32.5 against 15.6 / 15.8 / 17.0), from a K that
-     * falls with the rows (10240 x 5120 M = 2 / 3 / 4 8.7 / 11.8 / 13.6 against 11.6 / 11.7 / 11.8,
-     * 8704 x 5120 M = 4 / 6 10.9 / 12.9 against 10.9 / 11.2). */
-    const int long_pairs = M == 2 ? 48 : M == 3 ? 40 : M == 4 ? 34 : 20;
-    const bool stream_few = PAIR ? rows_smem(M, K, 0) > kMaxLds / 3 && tile_pairs >= 4 * device_cus()
-                                 : pairs > long_pairs && tile_pairs > device_cus();
-    if (M <= 8 && stream_few) {
-        const int st = launch_rows_stream<OUT, false>(x, M, w, s, out, N, K, stream, residual, cm);
+    if (PAIR) {
+        /* The row-tiled GEMM from 9 rows with six tile pairs a CU or more (M = 16: 2560 x 24576 10.9 us
+         * in the LDS-staged tile-pair form, 9.8 here; 1024 x 34816 8.2 / 7.6; below, 2560 x 19456 9.3 /
+         * 9.3, 4608 x 19456 14.3 / 13.2 but 1792 x 19456 7.6 / 7.8, 4608 x 8192 8.6 / 8.9), and from 6
+         * rows with four where fewer than four blocks of the few-row form, which stage all rows, fit a
+         * CU's LDS (M = 6: 4608 x 24576 18.7 / 14.7, 3584 x 19456 11.7 / 11.5; M = 8: 5120 x 34816
+         * 37.1 / 23.3, 3200 x 17152 11.9 / 10.5, against 2560 x 19456, four blocks, 8.6 / 9.1; five
+         * rows of 5120 x 34816 23.2 / 23.3). */
+        const int cus = device_cus();
+        if (M > 8 ? tile_pairs >= 6 * cus
+                  : M >= 6 && tile_pairs >= 4 * cus && rows_smem(M, K, 0) > kMaxLds / 4)
+            return launch_rows_gemm<OUT>(x, M, w, s, out, N, K, stream, nullptr, cm);
+    } else if (pairs > (M == 2 ? 48 : M == 3 ? 40 : M == 4 ? 32 : 20) && tile_pairs > device_cus()) {
+        /* A long K and more than one tile pair a CU: as launch_down_cm, whose sums these are (17408 x
+         * 5120 M = 2 / 3 / 8 19.5 / 20.7 / 32.5 us in the few-row form, 15.7 / 15 / 19 here; 8704 x 5120
+         * M = 4 / 8 10.2 / 13.5, 9.8 / 10.0), from a K that falls with the rows. */
+        const int st = launch_rows_stream<OUT_F32, false>(x, M, w, s, out, N, K, stream, residual);
         if (st <= 0) return st;
+        return launch_rows_gemm_cfg<OUT, 1, 2, 1, 8>(x, M, w, s, out, N, K, stream, residual, 0);
     }
-    /* A long K whose staged 9 to 16 rows would not fit LDS: the same kernel at more than one tile
-     * pair a CU, as in launch_down_cm (so the FFN's down projection and this one, row-major, sum in
-     * the same order), and at 16 rows (9728 x 2560 13.2 us registers-fed, 10.0 here; 14336 x 3584
-     * 19.9 against 13.6); registers-fed otherwise, and from M = 8 without the residual epilogue (C1
-     * down, whole calls: 20.5 us LDS-staged, 19.9 registers-fed; with the residual 23.3 / 23.6). */
+    /* a long K whose staged rows would not fit LDS: registers-fed from M = 8 (9 with the residual
+     * epilogue) to 15, as the FFN's own down projection (C1 down, whole calls: M = 8 LDS-staged 20.5
+     * us, 19.9 here); at 16 the row-tiled GEMM (9728 x 2560 13.2 registers-fed, 10.7 here) */
     const bool long_k = !PAIR && rows16_smem(M, K, 16) > kMaxLds;
-    if (M >= 9 && long_k && (M == 16 || tile_pairs > device_cus())) {
-        const int st = launch_rows_stream<OUT, false>(x, M, w, s, out, N, K, stream, residual, cm);
-        if (st <= 0) return st;
-    }
-    if (M >= (residual ? 9 : 8) && long_k) {
+    if (long_k && M >= (residual ? 9 : 8) && M <= 15) {
         const int st = launch_rows16x<OUT_F32>(x, M, w, s, out, N, K, stream, residual);
         if (st <= 0) return st;
     }
-    if (M > 8 && !residual) {
+    if (M > 8 && !residual && !long_k) {
         const int st = launch_rows16<PAIR, OUT_F32>(x, M, w, s, out, N, K, stream, cm);
         if (st <= 0) return st;
     }
-    /* 9 to 16 rows that the LDS-staged tile-pair form cannot hold: M = 9 / 16 5120 x 34816 62 / 65 us
-     * in the split-K MFMA form, 25 / 25 here; 4096 x 24576 34 / 37 against 17 / 18 */
-    if (M > 8) return launch_rows_stream<OUT, false>(x, M, w, s, out, N, K, stream, residual, cm);
+    /* what is left at 9 to 16 rows (the residual epilogue, K past the tile-pair form): 16 rows of
+     * 5120 x 5120 14.5 us in the split-K MFMA form, 8.7 here, of the gate/up pair 5120 x 34816 62.4 /
+     * 23.8 and 5120 x 8192 20.4 / 9.4 */
+    if (M > 8) return launch_rows_gemm<OUT>(x, M, w, s, out, N, K, stream, residual, cm);
     /* two rows on the matrix-core GEMV: the gate/up pair at 7 to 12 group pairs (four waves of
      * three) and the long K of the C1 down projection, 37 to 48 pairs (sixteen of three). Whole
      * C1 FFN call at M = 2: 12.58-12.66 us against 13.70-13.99 on this kernel's few-row form
@@ -2550,91 +2559,6 @@ MfmaPlan plan_mfma(int M, int N, int K) {
     p.partial_bytes = p.S > 1 ? (size_t)p.S * NT * 16 * M * sizeof(uint64_t) : 0;
     p.ncounters = p.S > 1 ? (size_t)NT : 0;
     return p;
-}
-
-/* The plan of rows_stream_kernel: the K split S (GS groups each) and the tile pairs a block that
- * take the least estimated time in one round of blocks, one a CU: 0.033 us a unit, 16 ns a KiB of
- * staged rows, 2.2 us for the combine of a split (fitted to M = 2..16 on 17 weights). S is at most
- * what the split-K MFMA form would use, so the scratch reserved for that serves here too. */
-struct StreamPlan {
-    int S, GS, TPB, grid;
-    size_t smem, partial_bytes, ncounters;
-};
-
-bool plan_stream(int M, int N, int K, bool split, StreamPlan *plan) {
-    const int G = K / 128, NT = (N / 8 + 1) / 2, cus = device_cus();
-    float least = 0.0f;
-    for (int s = 1; s <= (split ? std::min(8, (G + kGMax - 1) / kGMax) : 1); ++s) {
-        StreamPlan p{};
-        p.GS = (G + s - 1) / s;
-        p.S = (G + p.GS - 1) / p.GS;
-        p.TPB = (int)(((long long)NT * p.S + cus - 1) / cus);
-        p.grid = (NT + p.TPB - 1) / p.TPB * p.S;
-        p.smem = std::max(((size_t)p.GS * M * 256 + 1023) / 1024 * 1024, (size_t)32 * 1024);
-        if (p.smem > kMaxLds || p.TPB > 16) continue;
-        const float t = 0.033f * p.TPB * p.GS + 0.004f * p.GS * M + (p.S > 1 ? 2.2f : 0.0f);
-        if (least == 0.0f || t < least) {
-            least = t;
-            p.partial_bytes = p.S > 1 ? (size_t)p.S * NT * 16 * M * sizeof(uint64_t) : 0;
-            p.ncounters = p.S > 1 ? (size_t)NT : 0;
-            *plan = p;
-        }
-    }
-    return least > 0.0f;
-}
-
-/* Whether split_scratch can serve this size without allocating. */
-bool split_scratch_ready(size_t partial_bytes, size_t ncounters) {
-    if (t_fixed.active) return partial_bytes <= t_fixed.partial_bytes && ncounters <= t_fixed.ncounters;
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return false;
-    std::lock_guard<std::mutex> lock(g_scratch_mu);
-    return partial_bytes <= g_scratch[dev].partial_bytes && ncounters <= g_scratch[dev].ncounters;
-}
-
-/* Returns 1 when no plan fits, or when it would have to grow the scratch under graph capture (the
- * kernels it stands in for need none, so a first call that was captured before stays possible). */
-template <int OUT, bool CM>
-int launch_rows_stream(const uint16_t *x, int M, const uint8_t *w, const uint16_t *s, void *out, int N,
-                       int K, hipStream_t stream, uint16_t *residual, int cm) {
-    constexpr bool PAIR = OUT == kOutPairSilu;
-    StreamPlan p{};
-    if (!plan_stream(M, N, K, !PAIR, &p)) return 1;
-    uint64_t *partial = nullptr;
-    unsigned *counters = nullptr;
-    if (p.S > 1) {
-        if (!split_scratch_ready(p.partial_bytes, p.ncounters)) {
-            hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-            const int st = hip_status(hipStreamIsCapturing(stream, &cap), "hipStreamIsCapturing");
-            if (st) return st;
-            if (cap != hipStreamCaptureStatusNone || t_fixed.active) return 1;
-        }
-        const int st = split_scratch(p.partial_bytes, p.ncounters, &partial, &counters);
-        if (st) return st;
-    }
-    if (!PAIR && p.S > 1)
-        launch_k((rows_stream_kernel<OUT, CM, !PAIR>), dim3(p.grid), dim3(1024), p.smem, stream, x, M, w, s,
-                 out, N, K, p.TPB, p.S, p.GS, partial, counters, residual, cm);
-    else
-        launch_k((rows_stream_kernel<OUT, CM, false>), dim3(p.grid), dim3(1024), p.smem, stream, x, M, w, s,
-                 out, N, K, p.TPB, 1, p.GS, partial, counters, residual, cm);
-    return hip_status(hipGetLastError(), "rows stream launch");
-}
-
-/* The down projection of M rows of a chunk-major activation (64 to 192 groups of K). Up to one
- * tile pair a CU the registers-fed kernel; beyond, its blocks of a tile pair and 16 waves take a
- * second round, and one block a CU over its whole share is faster (M = 4 / 16: 8704 x 5120 12.7 / 14.4
- * against 10.6 / 12.0 us, 13824 x 5120 19.5 / 22.3 against 13.8 / 16.1; 9728 x 2560, 160 tile pairs,
- * 7.3 / 8.2 against 8.5 / 9.5; 12288 x 4096, 256, 9.7 / 11.4 against 10.5 / 13.4). */
-template <bool OUT_F32>
-int launch_down_cm(const uint16_t *act, int M, const uint8_t *w, const uint16_t *s, void *out, int N, int K,
-                   hipStream_t stream, uint16_t *residual = nullptr) {
-    if ((N / 8 + 1) / 2 > device_cus()) {
-        const int st = launch_rows_stream<OUT_F32 ? kOutF32 : kOutBf16, true>(act, M, w, s, out, N, K, stream,
-                                                                             residual, 0);
-        if (st <= 0) return st;
-    }
-    return launch_rows16x<OUT_F32, true>(act, M, w, s, out, N, K, stream, residual);
 }
 
 /* ---- The allocation-free scratch ------------------------------------------------------------

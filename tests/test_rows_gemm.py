@@ -1,6 +1,6 @@
-"""More than 16 activation rows: the row-tiled GEMM (rows_gemm_kernel) through each of its block
-shapes, at the edges of their row tiles, tile pairs and K steps, against the oracle. The
-tolerances are the suite's (assert_parity): 2 BF16 ULP and rel-L2 1e-3 of the double-accumulated
+"""The row-tiled GEMM (rows_gemm_kernel), where launch_rows and every call of more than 16 rows send
+work to it: each of its block shapes at the edges of their row tiles, tile pairs and K steps, against
+the oracle. The tolerances are the suite's (assert_parity): 2 BF16 ULP and rel-L2 1e-3 of the double-accumulated
 product."""
 
 import numpy as np
@@ -18,16 +18,21 @@ pytestmark = pytest.mark.gpu
 # pairs x groups a step) where the launcher's estimate picks it, with odd tile counts, rows that do
 # not fill the row tiles and K that does not fill the steps
 SHAPES = [
-    (17, 8, 128),
-    (33, 2568, 1664),    # 1 x 2 x 8
-    (33, 9736, 640),     # 1 x 4 x 4
-    (17, 9736, 640),     # 1 x 6 x 4
-    (17, 12296, 128),    # 2 x 4 x 4
-    (50, 12296, 640),    # 2 x 6 x 4
-    (33, 16424, 1920),   # 2 x 9 x 4
+    (17, 8, 128),        # 1 x 4 x 4
+    (17, 8, 5248),       # 1 x 1 x 16
+    (16, 520, 9856),     # 1 x 1 x 16, past the tile-pair form
+    (17, 8, 640),        # 1 x 2 x 8
+    (33, 2568, 2688),    # 1 x 3 x 8
+    (33, 2568, 1664),    # 1 x 4 x 4
+    (33, 5128, 640),     # 1 x 6 x 4
+    (33, 9736, 1152),    # 1 x 8 x 4
+    (33, 5128, 128),     # 1 x 10 x 2
+    (17, 12296, 640),    # 2 x 4 x 4
+    (120, 5128, 1152),   # 2 x 6 x 4
+    (50, 12296, 2688),   # 2 x 9 x 4
     (63, 19464, 640),    # 2 x 10 x 2
-    (127, 34824, 640),   # 4 x 10 x 2
-    (120, 24584, 768),   # 2 x 6 x 2
+    (120, 5128, 640),    # 2 x 6 x 2
+    (127, 19464, 640),   # 4 x 10 x 2
 ]
 
 
@@ -41,13 +46,28 @@ def test_linear_parity(cuda, m, n, k):
     assert_parity(out, oracle.gemm_bf16(x, p, s, n, k), f"gemm M={m} N={n} K={k}")
 
 
-@pytest.mark.parametrize("m,hidden,inter", [(17, 128, 128), (65, 640, 9728), (129, 640, 2176)])
+@pytest.mark.parametrize("m,hidden,inter", [
+    (9, 640, 12296), (16, 1152, 12288), (15, 5248, 4104),  # many tile pairs, or K past the tile-pair form
+    (6, 3584, 8196), (8, 2688, 8200),  # few rows whose staged copies leave a CU three blocks
+])
+def test_gate_up_parity(cuda, m, hidden, inter):
+    print(f"gate/up M={m} H={hidden} I={inter}", flush=True)
+    p, s = make_weight(2 * inter, hidden, seed=hidden + inter)
+    x = oracle.synth_activation(m, hidden, seed=m)
+    gu = w4a16.TiledWeight.from_artifact(p, s, 2 * inter, hidden, pair=True, device=cuda)
+    act = from_dev(w4a16.gate_up_silu(to_dev(x, cuda), gu))
+    want = oracle.silu_mul_packed(oracle.gemm_bf16(x, p, s, 2 * inter, hidden), m, inter)
+    assert_parity(act, want, f"gate/up M={m} H={hidden} I={inter}")
+
+
+@pytest.mark.parametrize("m,hidden,inter", [(17, 128, 128), (65, 640, 9728), (129, 640, 2176), (16, 256, 2176)])
 def test_ffn_forms(cuda, m, hidden, inter):
     """The gate/up pair and the down projection, each stage against the oracle on its own inputs
     (end to end a BF16 rounding of the intermediate that falls the other way moves an output by
     up to 2^-8 |act| |w|, which is no error of either stage); then the forms around them, which
     run the same kernels and have to agree bit for bit: the FP32 partial rounds to the BF16
-    output, and plan F2 is the MLP of the normed sum, with the residual gaining exactly it."""
+    output, and plan F2 is the MLP of the normed sum, with the residual gaining exactly it (at up to 16 rows
+    its down projection is another kernel than the MLP's, so there it is held to the oracle)."""
     print(f"ffn M={m} H={hidden} I={inter}", flush=True)
     gup, gus, dp, ds = make_ffn(hidden, inter, layer=40)
     gu = w4a16.TiledWeight.from_artifact(gup, gus, 2 * inter, hidden, pair=True, device=cuda)
@@ -69,5 +89,9 @@ def test_ffn_forms(cuda, m, hidden, inter):
     resd = to_dev(res, cuda)
     got = w4a16.mlp_int4_residual_norm(resd, to_dev(sub, cuda), to_dev(nw, cuda), 1, 1e-6, gu, dn)
     normed = w4a16.rmsnorm(to_dev(summed, cuda), to_dev(nw, cuda), 1, 1e-6)
-    assert torch.equal(got, w4a16.mlp_int4(normed, gu, dn))
+    if m > 16:
+        assert torch.equal(got, w4a16.mlp_int4(normed, gu, dn))
+    else:
+        act = from_dev(w4a16.gate_up_silu(normed, gu))
+        assert_parity(from_dev(got), oracle.gemm_bf16(act, dp, ds, hidden, inter), f"F2 down M={m} K={inter}")
     assert np.array_equal(from_dev(resd), oracle.residual_add_bf16(summed, from_dev(got)))
