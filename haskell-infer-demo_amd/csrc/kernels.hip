@@ -102,6 +102,38 @@ __device__ __forceinline__ float lane_sum32(float v) {
     return x + y;
 }
 
+template <int CTRL>
+__device__ __forceinline__ double dpp_f64(double v) {
+    const uint2 b = __builtin_bit_cast(uint2, v);
+    return __builtin_bit_cast(double, make_uint2((uint32_t)__builtin_amdgcn_update_dpp(0, (int)b.x, CTRL, 0xF, 0xF, true),
+                                                 (uint32_t)__builtin_amdgcn_update_dpp(0, (int)b.y, CTRL, 0xF, 0xF, true)));
+}
+
+/* Sum over the wave in FP64, for lane 63: within the rows of sixteen by DPP, then row 0 into 1, 2
+ * into 3, and 1 into 3 (the row broadcasts). VALU moves: six shuffles of a double are twelve round
+ * trips through the LDS crossbar, one behind the other. */
+__device__ __forceinline__ double wave_sum_f64(double v) {
+    v += dpp_f64<kDppQuadSwap1>(v);
+    v += dpp_f64<kDppQuadSwap2>(v);
+    v += dpp_f64<kDppRowRor4>(v);
+    v += dpp_f64<kDppRowRor8>(v);
+    v += dpp_f64<0x142>(v); /* row_bcast:15 */
+    v += dpp_f64<0x143>(v); /* row_bcast:31 */
+    return v;
+}
+
+/* RMSNorm's scale 1 / sqrt(sum / count + eps) from the FP64 sum of squares: v_rsq_f64 (good to
+ * 2^-24 or better) and one step of third order, so within a few FP64 roundings of the exact value as
+ * the division and the square root are, in a tenth of their instructions, which every wave of
+ * every block runs. A step from the infinities of rsq(0) and rsq(inf) is not a number; they stay. */
+__device__ __forceinline__ float norm_scale(double sum, double inv_count, float eps) {
+    const double v = fma(sum, inv_count, (double)eps);
+    const double r = __builtin_amdgcn_rsq(v);
+    const double e = fma(-v * r, r, 1.0);
+    const double better = fma(r * e, fma(e, 0.375, 0.5), r);
+    return (float)(e == e ? better : r);
+}
+
 /* Code pairs as BF16. In a tile word the pair (j = 2q, 2q+1) sits at bits 3 + 4q and 19 + 4q
  * (the word is stored rotated left by 3 bits, so the odd code of q = 3 wraps round to bits 31 and
  * 0-2): pair 0 already sits at bits 3-6 of its two 16-bit halves, pairs 1 and 2 get there by a
@@ -299,7 +331,7 @@ template <bool PAIR, bool OUT_F32, int TB, int SK, bool NORM, int NL>
 __global__ __launch_bounds__(TB * SK * 64) void gemv_tiles_kernel(
     const uint16_t *__restrict__ x, const uint8_t *__restrict__ wt,
     const uint16_t *__restrict__ st, void *__restrict__ out, int N, int K,
-    const uint16_t *__restrict__ norm_w, float norm_bias, float eps,
+    const uint16_t *__restrict__ norm_w, float norm_bias, float eps, double inv_k,
     const uint16_t *__restrict__ sub) {
     constexpr int W = TB * SK;
     /* the largest K this configuration is launched for: SK * NL group pairs */
@@ -403,14 +435,14 @@ __global__ __launch_bounds__(TB * SK * 64) void gemv_tiles_kernel(
                 ss = fma(hi, hi, ss);
             }
         }
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) ss += __shfl_xor(ss, o);
+        ss = wave_sum_f64(ss);
         double *dred = reinterpret_cast<double *>(red);
-        if (lane == 0) dred[wave] = ss;
+        if (lane == 63) dred[wave] = ss;
         __syncthreads();
         double total = 0.0;
+#pragma unroll
         for (int w = 0; w < W; ++w) total += dred[w];
-        const float rms = (float)(1.0 / sqrt(total / (double)K + (double)eps));
+        const float rms = norm_scale(total, inv_k, eps);
 #pragma unroll
         for (int it = 0; it < kXIters; ++it) {
             uint32_t w4[4] = {xv[it].x, xv[it].y, xv[it].z, xv[it].w};
@@ -1812,14 +1844,18 @@ __global__ __launch_bounds__(1024) void rows_stream_kernel(
 /* RMSNorm of each row (one block a row): BF16(x * rsqrt(sum x^2 / cols + eps) * (bias + w)),
  * FP32 arithmetic (reference csrc/kernels/flashinfer_norm.cu:22-76). Each thread holds CH
  * 8-value chunks of the row, all loaded before any use, so a row costs one load round trip;
- * cols % 8 == 0 and cols <= CH * 8 * 256 (the launcher checks). */
+ * cols % 8 == 0 and cols <= CH * 8 * blockDim.x <= 16384 (the launcher checks).
+ *
+ * What bounds it is latency: launch, one round trip, the chain of FP64 sums and the scale. As many
+ * threads as chunks (up to 1024) keep a thread's part of the chain to eight sums; 16 x 5120
+ * repeated in a graph 2.51 -> 2.26 us, 4 x 2560 2.23 -> 2.10, with norm_scale and wave_sum_f64 (2.0 of it
+ * is a launch that depends on the one before). */
 template <int CH>
-__global__ __launch_bounds__(256) void rmsnorm_kernel(uint16_t *__restrict__ out,
-                                                      uint16_t *x,
-                                                      const uint16_t *__restrict__ w, int cols,
-                                                      float bias, float eps,
-                                                      const uint16_t *sub) {
-    __shared__ double red[4];
+__global__ __launch_bounds__(1024) void rmsnorm_kernel(uint16_t *__restrict__ out, uint16_t *x,
+                                                       const uint16_t *__restrict__ w, int cols,
+                                                       float bias, float eps, double inv_cols,
+                                                       const uint16_t *sub) {
+    __shared__ double red[16];
     const int chunks = cols >> 3;
     const __amdgpu_buffer_rsrc_t xr = make_rsrc(x + (size_t)blockIdx.x * cols, (uint32_t)cols * 2);
     const __amdgpu_buffer_rsrc_t wr = make_rsrc(w, (uint32_t)cols * 2);
@@ -1828,7 +1864,7 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(uint16_t *__restrict__ out
     uint4 xv[CH], wv[CH], uv[CH];
 #pragma unroll
     for (int c = 0; c < CH; ++c) {
-        const int i = c * 256 + threadIdx.x;
+        const int i = c * (int)blockDim.x + threadIdx.x;
         xv[c] = buf_load16(xr, i < chunks ? (uint32_t)i * 16 : kOob);
         wv[c] = buf_load16(wr, i < chunks ? (uint32_t)i * 16 : kOob);
         uv[c] = buf_load16(ur, i < chunks ? (uint32_t)i * 16 : kOob);
@@ -1839,7 +1875,7 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(uint16_t *__restrict__ out
         uint4 *xrow = reinterpret_cast<uint4 *>(x + (size_t)blockIdx.x * cols);
 #pragma unroll
         for (int c = 0; c < CH; ++c) {
-            const int i = c * 256 + threadIdx.x;
+            const int i = c * (int)blockDim.x + threadIdx.x;
             xv[c] = make_uint4(bf16_add2(xv[c].x, uv[c].x), bf16_add2(xv[c].y, uv[c].y),
                                bf16_add2(xv[c].z, uv[c].z), bf16_add2(xv[c].w, uv[c].w));
             if (i < chunks) xrow[i] = xv[c];
@@ -1859,16 +1895,16 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(uint16_t *__restrict__ out
             ss = fma(hi, hi, ss);
         }
     }
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) ss += __shfl_xor(ss, o);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ss;
+    ss = wave_sum_f64(ss);
+    if ((threadIdx.x & 63) == 63) red[threadIdx.x >> 6] = ss;
     __syncthreads();
-    const double total = (red[0] + red[1]) + (red[2] + red[3]);
-    const float rms = (float)(1.0 / sqrt(total / (double)cols + (double)eps));
+    double total = 0.0;
+    for (int v = 0; v < (int)blockDim.x >> 6; ++v) total += red[v];
+    const float rms = norm_scale(total, inv_cols, eps);
     uint4 *orow = reinterpret_cast<uint4 *>(out + (size_t)blockIdx.x * cols);
 #pragma unroll
     for (int c = 0; c < CH; ++c) {
-        const int i = c * 256 + threadIdx.x;
+        const int i = c * (int)blockDim.x + threadIdx.x;
         const uint32_t x4[4] = {xv[c].x, xv[c].y, xv[c].z, xv[c].w};
         const uint32_t n4[4] = {wv[c].x, wv[c].y, wv[c].z, wv[c].w};
         uint32_t o4[4];
@@ -2093,11 +2129,12 @@ int launch_gemv_cfg(const uint16_t *x, const uint8_t *w, const uint16_t *s, void
     if (norm)
         launch_k((gemv_tiles_kernel<PAIR, OUT_F32, TB, SK, true, NL>),
                            dim3((tiles + TB - 1) / TB), dim3(TB * SK * 64), gemv_smem(K, TB * SK),
-                           stream, x, w, s, out, N, K, norm->w, norm->bias, norm->eps, norm->sub);
+                           stream, x, w, s, out, N, K, norm->w, norm->bias, norm->eps, 1.0 / K,
+                           norm->sub);
     else
         launch_k((gemv_tiles_kernel<PAIR, OUT_F32, TB, SK, false, NL>),
                            dim3((tiles + TB - 1) / TB), dim3(TB * SK * 64), gemv_smem(K, TB * SK),
-                           stream, x, w, s, out, N, K, nullptr, 0.0f, 0.0f, nullptr);
+                           stream, x, w, s, out, N, K, nullptr, 0.0f, 0.0f, 0.0, nullptr);
     return hip_status(hipGetLastError(), "gemv launch");
 }
 
@@ -2210,7 +2247,8 @@ int launch_gemv(const uint16_t *x, const uint8_t *w, const uint16_t *s, void *ou
     if (norm) {
         /* every block normalises all of x, yet the small-load shape still wins over fewer,
          * larger blocks (C1 norm + FFN medians: 2 x 2 x 5 14.9 us, 4 x 1 x 10 15.4, 4 x 2 x 5
-         * 15.5; the FFN alone 13.9) */
+         * 15.5; the FFN alone 13.9; since then norm_scale and wave_sum_f64 in place of FP64 divisions
+         * and shuffles took 0.48 us off every such FFN, 513 -> 496 us for 36 of plan F2) */
         if (pairs <= 10) return launch_gemv_cfg<PAIR, OUT_F32, 2, 2, 5>(x, w, s, out, N, K, stream, norm);
         if (pairs <= 12) return launch_gemv_cfg<PAIR, OUT_F32, 2, 2, 6>(x, w, s, out, N, K, stream, norm);
         return set_error(W4A16_ERR_CONFIG, "gemv: the RMSNorm prologue needs K <= 3072");
@@ -2924,14 +2962,16 @@ static int norm_args(const uint16_t *w, int style, float eps, int cols, int rows
 
 static int launch_rmsnorm(uint16_t *out, const uint16_t *x, const uint16_t *w, int cols, int rows,
                           float bias, float eps, hipStream_t s, const uint16_t *sub = nullptr) {
-    const int ch = (cols / 8 + 255) / 256;
-    if (cols % 8 || ch > 8)
+    const int chunks = cols / 8;
+    if (cols % 8 || chunks > 2048)
         return set_error(W4A16_ERR_CONFIG, "rmsnorm: cols=%d must be a multiple of 8 and <= 16384",
                          cols);
-    if (ch <= 1) launch_k(rmsnorm_kernel<1>, dim3(rows), dim3(256), 0, s, out, const_cast<uint16_t *>(x), w, cols, bias, eps, sub);
-    else if (ch <= 2) launch_k(rmsnorm_kernel<2>, dim3(rows), dim3(256), 0, s, out, const_cast<uint16_t *>(x), w, cols, bias, eps, sub);
-    else if (ch <= 4) launch_k(rmsnorm_kernel<4>, dim3(rows), dim3(256), 0, s, out, const_cast<uint16_t *>(x), w, cols, bias, eps, sub);
-    else launch_k(rmsnorm_kernel<8>, dim3(rows), dim3(256), 0, s, out, const_cast<uint16_t *>(x), w, cols, bias, eps, sub);
+    const int ch = chunks > 1024 ? 2 : 1;
+    const dim3 block((chunks + 64 * ch - 1) / (64 * ch) * 64);
+    if (ch == 1)
+        launch_k(rmsnorm_kernel<1>, dim3(rows), block, 0, s, out, const_cast<uint16_t *>(x), w, cols, bias, eps, 1.0 / cols, sub);
+    else
+        launch_k(rmsnorm_kernel<2>, dim3(rows), block, 0, s, out, const_cast<uint16_t *>(x), w, cols, bias, eps, 1.0 / cols, sub);
     return hip_status(hipGetLastError(), "rmsnorm launch");
 }
 
