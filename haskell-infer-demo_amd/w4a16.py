@@ -153,6 +153,12 @@ def _dev(t, nbytes, elem, what, device=None):
     `elem`-byte elements (BF16 bits as int16/bfloat16, FP32, u8) holding at least `nbytes`, on
     `device` when given. The kernels trust their extents, so a short or strided buffer would be
     read or written out of bounds on the GPU; this raises W4A16Error instead."""
+    try:
+        if (t.is_cuda and t.element_size() == elem and t.numel() * elem >= nbytes and t.is_contiguous()
+                and (device is None or t.device == device)):
+            return t.data_ptr()
+    except (AttributeError, TypeError):
+        pass  # no tensor: named below
     if not hasattr(t, "data_ptr") or not hasattr(t, "is_cuda"):
         raise W4A16Error(W4A16_ERR_CONFIG, f"{what}: expected a CUDA tensor, got {type(t).__name__}")
     if not t.is_cuda:
@@ -194,7 +200,8 @@ def _stream(stream):
     if stream is None:
         import torch
 
-        return torch.cuda.current_stream().cuda_stream
+        # the handle itself: building the Stream object around it takes longer than a kernel's launch
+        return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
     if isinstance(stream, int):
         return stream
     return stream.cuda_stream
