@@ -1515,6 +1515,16 @@ __device__ __forceinline__ void rows_store(float v, bool ok, int m, int tile, in
     }
 }
 
+/* A sum's rounding error grows with the length of its chains. Where a wave of rows_gemm_kernel or
+ * rows_stream_kernel has more products than kFoldFrom, their FOLD forms move its accumulators into
+ * second-level sums every kFold products, which keeps the error of FP32 partials at or below that of sixteen
+ * accumulators a column (17408 x 5120 against 64 bits, relative 2-norm, 33 / 128 / 200 rows: sixteen accumulators
+ * 1.68e-7 / 1.68e-7 / 1.67e-7, chains of 34, 34 and 68 1.80e-7 / 1.79e-7 / 2.04e-7). Up to 8 row-major rows
+ * the shorter chains of gemv_rows_kernel are the measure, with kFoldFew (2 rows 1.61e-7 there, in chains of
+ * 17 1.66e-7, here 1.59e-7). The gate/up pair, which ends in BF16, keeps up to kFoldFromPair: folding costs a block the
+ * LDS that lets the next one start (5120 x 34816 at 128 rows 97 -> 104 us). */
+constexpr int kFold = 16, kFoldFrom = 17, kFoldFew = 6, kFoldFromPair = 20;
+
 /* Rows by tiles of 16: a block of WN x WK waves owns WN * TPW tile pairs and 16 MT activation rows
  * over all of K. In each step wave (wn, wk) takes group c WK + wk of its TPW tile pairs from memory
  * and unpacks it once for all MT row tiles; the block's rows of the WK groups are staged in LDS,
@@ -1538,16 +1548,18 @@ __device__ __forceinline__ void rows_store(float v, bool ok, int m, int tile, in
  * 12.8 / 18.0 / 28.9 us; 5120 x 34816 M = 16 / 32 / 64 / 128 61 / 120 / 241 / 480 -> 23.5 / 29.7 / 49 / 97;
  * down 9728 x 2560 M = 32 / 64 / 128 24.2 / 35.9 / 57.4 -> 12.5 / 14.3 / 22.3; 17408 x 5120 M = 16 /
  * 32 / 64 / 128 24.8 / 61 / 100 / 194 -> 20.6 / 23.7 / 34.9 / 50.2. */
-template <int OUT, int MT, int TPW, int WN, int WK, bool CM>
+template <int OUT, int MT, int TPW, int WN, int WK, bool CM, bool FOLD>
 __global__ __launch_bounds__(WN * WK * 64) void rows_gemm_kernel(
     const uint16_t *__restrict__ x, int M, const uint8_t *__restrict__ wt,
-    const uint16_t *__restrict__ st, void *__restrict__ out, int N, int K, int Y, uint16_t *residual, int cm) {
+    const uint16_t *__restrict__ st, void *__restrict__ out, int N, int K, int Y, uint16_t *residual, int cm,
+    int period) {
     static_assert(!CM || MT == 1, "a chunk-major activation has at most 16 rows");
     constexpr int T = WN * WK * 64;
     constexpr int ROWS = 16 * MT;
     constexpr int CHUNKS = WK * ROWS * 16; /* 16-byte chunks of one staged step */
     constexpr int XL = (CHUNKS + T - 1) / T;
-    extern __shared__ uint4 smem4[]; /* two steps; then the wave reduction */
+    constexpr int TILES = MT * TPW;
+    extern __shared__ uint4 smem4[]; /* two steps; then, or with FOLD behind them, the wave reduction */
     const int G = K >> 7;
     const int tiles = N >> 3;
     const int NT = (tiles + 1) >> 1;
@@ -1615,6 +1627,8 @@ __global__ __launch_bounds__(WN * WK * 64) void rows_gemm_kernel(
     };
 
     const int steps = (G + WK - 1) / WK;
+    f32x4_t *red = reinterpret_cast<f32x4_t *>(smem4) + (FOLD ? 2 * CHUNKS : 0); /* [WN][TILES][WK][64 lanes] */
+    f32x4_t *mine = red + (wn * TILES * WK + wk) * 64 + lane;                    /* this lane's, 64 WK apart */
     load_x(0);
     __builtin_amdgcn_sched_barrier(0);
     load_w(0);
@@ -1629,6 +1643,7 @@ __global__ __launch_bounds__(WN * WK * 64) void rows_gemm_kernel(
 #pragma unroll
         for (int p = 0; p < TPW; ++p) acc[mt][p] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
 
+    int since = 0; /* steps in acc */
     for (int c0 = 0; c0 < steps; c0 += 2) {
 #pragma unroll
         for (int v = 0; v < 2; ++v) { /* the buffer of step c */
@@ -1671,17 +1686,30 @@ __global__ __launch_bounds__(WN * WK * 64) void rows_gemm_kernel(
             stage_x((v + 1) & 1);
             __syncthreads();
         }
+        if (FOLD && (since += 2) == period && c0 + 2 < steps) { /* the slots are this lane's own: no barrier */
+            since = 0;
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+                for (int p = 0; p < TPW; ++p) {
+                    f32x4_t *slot = mine + (mt * TPW + p) * WK * 64;
+                    if (c0 >= period) acc[mt][p] += *slot;
+                    *slot = acc[mt][p];
+                    acc[mt][p] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+                }
+        }
     }
 
     /* the WK waves of a column group meet in LDS; then the block's waves take D register j of tile t,
      * a rolled loop (unrolled over tiles and registers this code was several times the main loop) */
-    constexpr int TILES = MT * TPW;
-    f32x4_t *red = reinterpret_cast<f32x4_t *>(smem4); /* [WN][TILES][WK][64 lanes] */
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-        for (int p = 0; p < TPW; ++p)
-            red[((wn * TILES + mt * TPW + p) * WK + wk) * 64 + lane] = acc[mt][p];
+        for (int p = 0; p < TPW; ++p) {
+            f32x4_t *slot = mine + (mt * TPW + p) * WK * 64;
+            if (FOLD) acc[mt][p] += *slot; /* more than `period` steps: written before */
+            *slot = acc[mt][p];
+        }
     __syncthreads();
     for (int i = wave; i < WN * TILES * 4; i += WN * WK) {
         const int j = i & 3, t = i >> 2;
@@ -1712,7 +1740,7 @@ __global__ __launch_bounds__(WN * WK * 64) void rows_gemm_kernel(
  * the gate/up kernel the combine's mailbox costs up to 10 us (10240 x 5120 M = 4 22.8 us with three
  * splits, 11.0 with none). Down projections between gate/up calls, before / here: 17408 x 5120 M = 4
  * 20.6 -> 14.9 us; 10240 x 5120 M = 4 / 8 12.5 / 12.7 -> 10.4 / 11.1; 8704 x 5120 M = 8 11.3 -> 10.0. */
-template <bool OUT_F32, bool CM>
+template <bool OUT_F32, bool CM, bool FOLD>
 __global__ __launch_bounds__(1024) void rows_stream_kernel(
     const uint16_t *__restrict__ x, int M, const uint8_t *__restrict__ wt,
     const uint16_t *__restrict__ st, void *__restrict__ out, int N, int K, int TPB, uint16_t *residual) {
@@ -1778,7 +1806,8 @@ __global__ __launch_bounds__(1024) void rows_stream_kernel(
     __syncthreads();
 
     const uint4 offs = make_uint4(0xBF40BF40u, 0xBF40BF40u, 0xBF40BF40u, 0xBF40BF40u);
-    f32x4_t acc = {0.0f, 0.0f, 0.0f, 0.0f}, first = acc;
+    f32x4_t acc = {0.0f, 0.0f, 0.0f, 0.0f}, first = acc, folded = acc;
+    int since = 0; /* units in acc */
     const int arow = min(n, M - 1);
     int cu = u0, cg = u0 - p0 * G;
     const int cnt = u1 - u0;
@@ -1800,11 +1829,21 @@ __global__ __launch_bounds__(1024) void rows_stream_kernel(
 #pragma unroll
                 for (int j = 0; j < 4; ++j) acc[j] = fmaf(sc, d[j], acc[j]);
                 ++cu;
+                if (FOLD && ++since == kFoldFew) {
+                    since = 0;
+                    folded += acc;
+                    acc = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+                }
                 if (++cg == G) { /* the end of a tile pair: the wave's range may go on into the next */
                     cg = 0;
                     if (cu < u1) {
                         first = acc;
                         acc = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+                        if (FOLD) {
+                            since = 0;
+                            first += folded;
+                            folded = acc;
+                        }
                     }
                 }
             }
@@ -1813,6 +1852,7 @@ __global__ __launch_bounds__(1024) void rows_stream_kernel(
     }
     __syncthreads();
     f32x4_t *red = reinterpret_cast<f32x4_t *>(smem4); /* [16 waves][its first, its second pair][64 lanes] */
+    if (FOLD) acc += folded;
     const bool two = cnt > 0 && (u1 - 1) / G != p0;
     red[(wave * 2 + 0) * 64 + lane] = two ? first : acc;
     red[(wave * 2 + 1) * 64 + lane] = acc;
@@ -2345,8 +2385,11 @@ template <int OUT, int MT, int TPW, int WN, int WK, bool CM = false>
 int launch_rows_gemm_cfg(const uint16_t *x, int M, const uint8_t *w, const uint16_t *s, void *out, int N,
                          int K, hipStream_t stream, uint16_t *residual, int cm) {
     constexpr size_t stage = (size_t)2 * WK * 16 * MT * 256, reduce = (size_t)WK * WN * MT * TPW * 1024;
-    constexpr size_t smem = stage > reduce ? stage : reduce;
-    static_assert(smem <= kMaxLds, "the two staged steps and the reduction fit a block's LDS");
+    static_assert(stage + reduce <= kMaxLds, "the two staged steps and the reduction fit a block's LDS");
+    const bool few = M <= 8 && !CM;
+    const int period = few ? kFoldFew : kFold;
+    const bool fold = K / 128 > (few ? kFoldFew : OUT == kOutPairSilu ? kFoldFromPair : kFoldFrom) * WK;
+    const size_t smem = fold ? stage + reduce : std::max(stage, reduce);
     constexpr size_t elem = OUT == kOutF32 ? 4 : 2;
     const int cols = (((N / 8 + 1) / 2 + WN * TPW - 1) / (WN * TPW) + 7) / 8 * 8;
     /* a launch of at most 2^21 blocks (a grid holds fewer than 2^32 threads): in practice all rows */
@@ -2354,9 +2397,10 @@ int launch_rows_gemm_cfg(const uint16_t *x, int M, const uint8_t *w, const uint1
     for (int m0 = 0; m0 < M; m0 += most) {
         const int rows = std::min(M - m0, most), slices = (rows + 16 * MT - 1) / (16 * MT);
         const size_t o = (size_t)m0 * (OUT == kOutPairSilu ? N / 2 : N);
-        launch_k((rows_gemm_kernel<OUT, MT, TPW, WN, WK, CM>), dim3((unsigned)cols * slices),
-                 dim3(WN * WK * 64), smem, stream, x + (size_t)m0 * K, rows, w, s,
-                 static_cast<char *>(out) + o * elem, N, K, slices, residual ? residual + o : nullptr, cm);
+        launch_k((fold ? rows_gemm_kernel<OUT, MT, TPW, WN, WK, CM, true>
+                       : rows_gemm_kernel<OUT, MT, TPW, WN, WK, CM, false>),
+                 dim3((unsigned)cols * slices), dim3(WN * WK * 64), smem, stream, x + (size_t)m0 * K, rows, w, s,
+                 static_cast<char *>(out) + o * elem, N, K, slices, residual ? residual + o : nullptr, cm, period);
         const int st = hip_status(hipGetLastError(), "rows gemm launch");
         if (st) return st;
     }
@@ -2441,8 +2485,10 @@ int launch_rows_stream(const uint16_t *x, int M, const uint8_t *w, const uint16_
     /* the rows, then in their place two partial sums a wave */
     const size_t smem = std::max(((size_t)(K / 128) * M * 256 + 1023) / 1024 * 1024, (size_t)32 * 1024);
     if (M > 16 || TPB > 16 || smem > kMaxLds) return 1;
-    launch_k((rows_stream_kernel<OUT_F32, CM>), dim3((tile_pairs + TPB - 1) / TPB), dim3(1024), smem, stream,
-             x, M, w, s, out, N, K, TPB, residual);
+    /* a wave has TPB G / 16 units, of one tile pair at most G */
+    const bool fold = std::min(K / 128, (TPB * (K / 128) + 15) / 16) > (CM ? kFoldFrom : kFoldFew);
+    launch_k((fold ? rows_stream_kernel<OUT_F32, CM, true> : rows_stream_kernel<OUT_F32, CM, false>),
+             dim3((tile_pairs + TPB - 1) / TPB), dim3(1024), smem, stream, x, M, w, s, out, N, K, TPB, residual);
     return hip_status(hipGetLastError(), "rows stream launch");
 }
 
