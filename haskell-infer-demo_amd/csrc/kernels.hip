@@ -52,6 +52,7 @@
 #include <mutex>
 
 #include "common.h"
+#include "rows_shape.h"
 
 using namespace w4a16;
 
@@ -2407,43 +2408,11 @@ int launch_rows_gemm_cfg(const uint16_t *x, int M, const uint8_t *w, const uint1
     return W4A16_OK;
 }
 
-/* rows_gemm_kernel in the block shape whose estimated time is least: base + steps * (first + more *
- * (rounds - 1)), with steps = ceil(groups / WK) and rounds the blocks of the fullest CU, counted on
- * the fullest XCD (column blocks go round the eight XCDs, a column block's row slices stay on one).
- * A shape's three constants are a least-squares fit (relative error 3 to 8 %) to its times over 22
- * weights, K 1024 to 17408 and N 1024 to 34816, and 16 to 128 rows; the choice is on average within
- * 1 % of the best shape there and never more than 20 % off. No shape serves all: at 32 rows
- * 9728 x 2560 takes 12.0 us as 1 x 2 x 8 (row tiles x tile pairs x groups a step) and 20 as 2 x 6 x
- * 4, which takes 12.1 us where 2560 x 19456 takes 17 as 1 x 2 x 8. */
+/* rows_gemm_kernel in the block shape that rows_shape picks. */
 template <int OUT>
 int launch_rows_gemm(const uint16_t *x, int M, const uint8_t *w, const uint16_t *s, void *out, int N,
                      int K, hipStream_t stream, uint16_t *residual = nullptr, int cm = 0) {
-    struct Shape {
-        int rows, tile_pairs, groups; /* a block's rows / 16 and tile pairs, groups a step */
-        float base, first, more;      /* us */
-    };
-    static constexpr Shape shapes[] = {
-        {1, 1, 16, 6.02f, 0.60f, 2.11f}, {1, 2, 8, 4.05f, 0.77f, 1.33f},  {1, 3, 8, 4.40f, 0.89f, 1.55f},
-        {1, 4, 4, 3.62f, 0.63f, 0.65f},  {1, 6, 4, 4.13f, 0.80f, 1.18f},  {1, 8, 4, 4.18f, 0.98f, 1.42f},
-        {1, 10, 2, 4.13f, 0.65f, 0.85f}, {2, 4, 4, 4.13f, 0.94f, 1.34f},  {2, 6, 4, 5.07f, 1.09f, 1.77f},
-        {2, 9, 4, 6.50f, 1.45f, 2.33f},  {2, 10, 2, 5.46f, 0.94f, 1.31f}, {2, 6, 2, 4.85f, 0.74f, 0.64f},
-        {4, 10, 2, 6.89f, 1.67f, 2.32f},
-    };
-    const int G = K / 128, tile_pairs = (N / 8 + 1) / 2, xcd_cus = std::max(1, device_cus() / 8);
-    int best = 0;
-    float least = 0.0f;
-    for (int i = 0; i < (int)(sizeof(shapes) / sizeof(shapes[0])); ++i) {
-        const Shape &c = shapes[i];
-        const long long blocks = ((long long)(tile_pairs + c.tile_pairs - 1) / c.tile_pairs + 7) / 8 *
-                                 ((M + 16 * c.rows - 1) / (16 * c.rows));
-        const float rounds = (float)((blocks + xcd_cus - 1) / xcd_cus);
-        const float t = c.base + (float)((G + c.groups - 1) / c.groups) * (c.first + c.more * (rounds - 1.0f));
-        if (i == 0 || t < least) {
-            best = i;
-            least = t;
-        }
-    }
-    switch (best) {
+    switch (rows_shape(M, N, K, device_cus())) {
         case 0: return launch_rows_gemm_cfg<OUT, 1, 1, 1, 16>(x, M, w, s, out, N, K, stream, residual, cm);
         case 1: return launch_rows_gemm_cfg<OUT, 1, 2, 1, 8>(x, M, w, s, out, N, K, stream, residual, cm);
         case 2: return launch_rows_gemm_cfg<OUT, 1, 3, 1, 8>(x, M, w, s, out, N, K, stream, residual, cm);
@@ -2531,10 +2500,12 @@ int launch_rows(const uint16_t *x, int M, const uint8_t *w, const uint16_t *s, v
     } else if (pairs > (M == 2 ? 48 : M == 3 ? 40 : M == 4 ? 32 : 20) && tile_pairs > device_cus()) {
         /* A long K and more than one tile pair a CU: as launch_down_cm, whose sums these are (17408 x
          * 5120 M = 2 / 3 / 8 19.5 / 20.7 / 32.5 us in the few-row form, 15.7 / 15 / 19 here; 8704 x 5120
-         * M = 4 / 8 10.2 / 13.5, 9.8 / 10.0), from a K that falls with the rows. */
+         * M = 4 / 8 10.2 / 13.5, 9.8 / 10.0), from a K that falls with the rows. Rows that do not fit LDS
+         * take the row-tiled GEMM in the shape that suits N (16 rows: 12288 x 12288 26.1 us as 1 x 2 x 8, 19.4 so,
+         * 17408 x 17408 54.9 / 38.4). */
         const int st = launch_rows_stream<OUT_F32, false>(x, M, w, s, out, N, K, stream, residual);
         if (st <= 0) return st;
-        return launch_rows_gemm_cfg<OUT, 1, 2, 1, 8>(x, M, w, s, out, N, K, stream, residual, 0);
+        return launch_rows_gemm<OUT>(x, M, w, s, out, N, K, stream, residual);
     }
     /* a long K whose staged rows would not fit LDS: registers-fed from M = 8 (9 with the residual
      * epilogue) to 15, as the FFN's own down projection (C1 down, whole calls: M = 8 LDS-staged 20.5

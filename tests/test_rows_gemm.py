@@ -95,3 +95,20 @@ def test_ffn_forms(cuda, m, hidden, inter):
         act = from_dev(w4a16.gate_up_silu(normed, gu))
         assert_parity(from_dev(got), oracle.gemm_bf16(act, dp, ds, hidden, inter), f"F2 down M={m} K={inter}")
     assert np.array_equal(from_dev(resd), oracle.residual_add_bf16(summed, from_dev(got)))
+
+
+@pytest.mark.parametrize("m,n,k,more", [(16, 28672, 8192, 17), (11, 14344, 8192, 24)])
+def test_few_rows_take_the_shape_of_their_width(cuda, m, n, k, more):
+    """A long K whose rows rows_stream_kernel cannot hold runs in the shape that N asks for, as more rows do:
+    the estimate gives both row counts four groups a step, so the shared rows have the same sums."""
+    print(f"gemm M={m} and {more} N={n} K={k}", flush=True)
+    gen = torch.Generator().manual_seed(n)
+    packed = torch.randint(0, 256, (n, k // 2), generator=gen, dtype=torch.uint8)
+    scales = (0.002 + 0.002 * torch.rand(n, k // 128, generator=gen)).to(torch.bfloat16).view(torch.int16)
+    w = w4a16.TiledWeight.from_device_artifact(packed.to(cuda), scales.to(cuda), n, k)
+    x = torch.randn(more, k, generator=gen).to(torch.bfloat16).to(cuda)
+    few = w4a16.gemm_int4_bf16(x[:m], w)
+    assert torch.equal(few, w4a16.gemm_int4_bf16(x, w)[:m])
+    dense = w.dequantize().double()
+    assert_parity(from_dev(few.view(torch.int16)), from_dev((x[:m].double() @ dense.T).to(torch.bfloat16).view(torch.int16)),
+                  f"gemm M={m} N={n} K={k}")

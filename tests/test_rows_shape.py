@@ -1,0 +1,56 @@
+"""The block shapes of the row-tiled GEMM's GPU cases are the ones the launcher picks for them on 256 CUs, and all
+shapes are among them. rows_shape.h is host code; it is compiled here as it stands."""
+
+import os
+import shutil
+import subprocess
+
+import pytest
+
+from test_rows_gemm import SHAPES
+
+CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "haskell-infer-demo_amd", "csrc")
+
+MAIN = """
+#include <cstdio>
+#include <cstdlib>
+#include "rows_shape.h"
+int main(int argc, char **argv) {
+    for (int i = 1; i + 2 < argc; i += 3) {
+        const auto &s = w4a16::kRowsShapes[w4a16::rows_shape(atoi(argv[i]), atoi(argv[i + 1]), atoi(argv[i + 2]), 256)];
+        std::printf("%d %d %d\\n", s.rows, s.tile_pairs, s.groups);
+    }
+    std::printf("%d\\n", (int)(sizeof(w4a16::kRowsShapes) / sizeof(w4a16::kRowsShapes[0])));
+}
+"""
+
+# row tiles x tile pairs x groups a step of each of SHAPES
+PICKED = [(1, 4, 4), (1, 1, 16), (1, 1, 16), (1, 2, 8), (1, 3, 8), (1, 4, 4), (1, 6, 4), (1, 8, 4), (1, 10, 2),
+          (2, 4, 4), (2, 6, 4), (2, 9, 4), (2, 10, 2), (2, 6, 2), (4, 10, 2)]
+
+
+@pytest.fixture(scope="module")
+def picked(tmp_path_factory):
+    if shutil.which("g++") is None:
+        pytest.skip("g++ is not available")
+    d = tmp_path_factory.mktemp("shape")
+    (d / "main.cpp").write_text(MAIN)
+    subprocess.run(["g++", "-std=c++17", f"-I{CSRC}", "-o", str(d / "shape"), str(d / "main.cpp")], check=True)
+
+    def ask(sizes):
+        argv = [str(v) for size in sizes for v in size]
+        lines = subprocess.run([str(d / "shape"), *argv], check=True, capture_output=True, text=True).stdout.split("\n")
+        return [tuple(map(int, line.split())) for line in lines[:len(sizes)]], int(lines[len(sizes)])
+
+    return ask
+
+
+def test_shapes_of_the_gpu_cases(picked):
+    shapes, count = picked(SHAPES)
+    assert shapes == PICKED
+    assert len(set(shapes)) == count
+
+
+def test_few_rows_and_more_share_their_groups_a_step(picked):
+    shapes, _ = picked([(16, 28672, 8192), (17, 28672, 8192), (11, 14344, 8192), (24, 14344, 8192)])
+    assert [s[2] for s in shapes] == [4, 4, 4, 4]
