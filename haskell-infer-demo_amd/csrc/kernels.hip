@@ -64,7 +64,6 @@ constexpr int kMaxLoads = 12;     /* group pairs one wave holds when it takes a 
 constexpr int kMaxGemvK = 30464;  /* block-staged GEMV: 2K bytes of activation + sums in 64 KiB */
 constexpr int kMaxRowK = 49152;   /* M = 1: the reference's limit (K * 2 <= 96 KiB of staging) */
 constexpr int kMaxAnyK = 1 << 20; /* M > 1 (the MFMA form stages only its K range) */
-constexpr size_t kMaxLds = 163840; /* LDS a block can allocate on gfx950 */
 
 /* Cross-lane moves on the DPP path (a VALU operand modifier, no LDS round trip). quad_perm
  * patterns permute within groups of four lanes, row_ror:n rotates within rows of sixteen, and
@@ -2302,13 +2301,6 @@ int launch_gemv(const uint16_t *x, const uint8_t *w, const uint16_t *s, void *ou
     return launch_gemv_cfg<PAIR, OUT_F32, 1, 16, 8>(x, w, s, out, N, K, stream);
 }
 
-/* Few-row kernel: LDS for both groups of every pair of the M rows (whole 1 KiB load
- * instructions) and the wave reduction. */
-size_t rows_smem(int M, int K, int waves) {
-    const int P = (K / 128 + 1) / 2;
-    return (size_t)((P * 32 * M + 63) / 64) * 1024 + (size_t)waves * 256;
-}
-
 template <bool PAIR, bool OUT_F32, int TB, int SK, int NL>
 int launch_rows_mi(const uint16_t *x, int M, const uint8_t *w, const uint16_t *s, void *out,
                    int N, int K, hipStream_t stream, uint16_t *residual = nullptr, int cm = 0) {
@@ -2497,12 +2489,18 @@ int launch_rows(const uint16_t *x, int M, const uint8_t *w, const uint16_t *s, v
         if (M > 8 ? tile_pairs >= 6 * cus
                   : M >= 6 && tile_pairs >= 4 * cus && rows_smem(M, K, 0) > kMaxLds / 4)
             return launch_rows_gemm<OUT>(x, M, w, s, out, N, K, stream, nullptr, cm);
-    } else if (pairs > (M == 2 ? 48 : M == 3 ? 40 : M == 4 ? 32 : 20) && tile_pairs > device_cus()) {
-        /* A long K and more than one tile pair a CU: as launch_down_cm, whose sums these are (17408 x
-         * 5120 M = 2 / 3 / 8 19.5 / 20.7 / 32.5 us in the few-row form, 15.7 / 15 / 19 here; 8704 x 5120
-         * M = 4 / 8 10.2 / 13.5, 9.8 / 10.0), from a K that falls with the rows. Rows that do not fit LDS
-         * take the row-tiled GEMM in the shape that suits N (16 rows: 12288 x 12288 26.1 us as 1 x 2 x 8, 19.4 so,
-         * 17408 x 17408 54.9 / 38.4). */
+    }
+    /* 9 rows and more in the LDS-staged tile-pair form where it can hold K, also past one tile pair a CU (9 / 13
+     * rows of 5248 x 5120 6.9 / 7.2 us, 8.3 / 8.7 in rows_stream_kernel) */
+    const bool long_k = !PAIR && rows16_smem(M, K, 16) > kMaxLds;
+    if (M > 8 && !residual && !long_k) {
+        const int st = launch_rows16<PAIR, OUT_F32>(x, M, w, s, out, N, K, stream, cm);
+        if (st <= 0) return st;
+    }
+    /* a long K and more than one tile pair a CU, as launch_down_cm; rows that do not fit LDS take the
+     * row-tiled GEMM in the shape that suits N (16 rows: 12288 x 12288 26.1 us as 1 x 2 x 8, 19.4 so,
+     * 17408 x 17408 54.9 / 38.4) */
+    if (!PAIR && rows_streams(M, N, K, device_cus())) {
         const int st = launch_rows_stream<OUT_F32, false>(x, M, w, s, out, N, K, stream, residual);
         if (st <= 0) return st;
         return launch_rows_gemm<OUT>(x, M, w, s, out, N, K, stream, residual);
@@ -2510,13 +2508,8 @@ int launch_rows(const uint16_t *x, int M, const uint8_t *w, const uint16_t *s, v
     /* a long K whose staged rows would not fit LDS: registers-fed from M = 8 (9 with the residual
      * epilogue) to 15, as the FFN's own down projection (C1 down, whole calls: M = 8 LDS-staged 20.5
      * us, 19.9 here); at 16 the row-tiled GEMM (9728 x 2560 13.2 registers-fed, 10.7 here) */
-    const bool long_k = !PAIR && rows16_smem(M, K, 16) > kMaxLds;
     if (long_k && M >= (residual ? 9 : 8) && M <= 15) {
         const int st = launch_rows16x<OUT_F32>(x, M, w, s, out, N, K, stream, residual);
-        if (st <= 0) return st;
-    }
-    if (M > 8 && !residual && !long_k) {
-        const int st = launch_rows16<PAIR, OUT_F32>(x, M, w, s, out, N, K, stream, cm);
         if (st <= 0) return st;
     }
     /* what is left at 9 to 16 rows (the residual epilogue, K past the tile-pair form): 16 rows of

@@ -1,12 +1,16 @@
 /*
- * rows_shape.h - the block shapes of rows_gemm_kernel and the choice between them (host only).
+ * rows_shape.h - host-only rules of the multi-row dispatch: the block shapes of rows_gemm_kernel and the choice
+ * between them, and which linears of a few rows rows_stream_kernel takes.
  */
 #ifndef W4A16_ROWS_SHAPE_H
 #define W4A16_ROWS_SHAPE_H
 
 #include <algorithm>
+#include <cstddef>
 
 namespace w4a16 {
+
+constexpr std::size_t kMaxLds = 163840; /* LDS a block can allocate on gfx950 */
 
 struct RowsShape {
     int rows, tile_pairs, groups; /* a block's rows / 16 and tile pairs, groups a step */
@@ -45,6 +49,30 @@ inline int rows_shape(int M, int N, int K, int cus) {
         }
     }
     return best;
+}
+
+/* The few-row kernel's LDS: both groups of every pair of the M rows (whole 1 KiB load instructions) and the
+ * wave reduction. */
+inline std::size_t rows_smem(int M, int K, int waves) {
+    const int P = (K / 128 + 1) / 2;
+    return (std::size_t)((P * 32 * M + 63) / 64) * 1024 + (std::size_t)waves * 256;
+}
+
+/* Whether an N x K linear of M <= 16 row-major rows that no LDS-staged tile-pair kernel takes runs on
+ * rows_stream_kernel (or past its LDS on the row-tiled GEMM): with more than one tile pair a CU, from a K that falls
+ * with the rows (17408 x 5120 M = 2 / 3 / 8 18.9 / 19.3 / 30.9 us in the few-row form, 17.8 / 17.6 / 21.3 there;
+ * 8704 x 5120 M = 5 / 8 11.9 / 12.6, 10.5 / 11.0). With up to two tile pairs a CU the few-row form keeps 4 rows a
+ * little longer (8704 x 5120 10.3 / 10.6) and up to 64 KB of rows (5 rows of 5248 x 4224 7.3 / 7.8, of 6144 x 8192
+ * 9.2 / 9.5, but 6 of 6144 x 5120 8.4 / 8.2, and 5 of 5248 x 9728 11.5 / 10.0); and just past one tile pair a CU, where
+ * the streamed kernel leaves half of the CUs without a block, as long as two blocks of it fit a CU (5 rows of
+ * 7168 x 4104 8.2 / 9.0). */
+inline bool rows_streams(int M, int N, int K, int cus) {
+    const int pairs = (K / 128 + 1) / 2, tile_pairs = (N / 8 + 1) / 2;
+    const bool narrow = tile_pairs <= 2 * cus;
+    if (tile_pairs <= cus || pairs <= (M == 2 ? 48 : M == 3 ? 40 : M == 4 ? (narrow ? 36 : 32) : 20)) return false;
+    const std::size_t staged = rows_smem(M, K, 16);
+    if (M >= 5 && narrow && staged <= 68 * 1024) return false; /* the rows and the waves' sums */
+    return !(M >= 4 && tile_pairs < cus + cus / 32 && staged <= kMaxLds / 2);
 }
 
 }  // namespace w4a16

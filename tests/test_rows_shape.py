@@ -1,5 +1,6 @@
-"""The block shapes of the row-tiled GEMM's GPU cases are the ones the launcher picks for them on 256 CUs, and all
-shapes are among them. rows_shape.h is host code; it is compiled here as it stands."""
+"""The host-only rules of the multi-row dispatch on 256 CUs: the block shapes of the row-tiled GEMM's GPU cases are
+the ones the launcher picks, with all shapes among them, and the linears of a few rows go to the kernel that
+measured faster. rows_shape.h is compiled here as it stands."""
 
 import os
 import shutil
@@ -18,7 +19,8 @@ MAIN = """
 int main(int argc, char **argv) {
     for (int i = 1; i + 2 < argc; i += 3) {
         const auto &s = w4a16::kRowsShapes[w4a16::rows_shape(atoi(argv[i]), atoi(argv[i + 1]), atoi(argv[i + 2]), 256)];
-        std::printf("%d %d %d\\n", s.rows, s.tile_pairs, s.groups);
+        std::printf("%d %d %d %d\\n", s.rows, s.tile_pairs, s.groups,
+                    (int)w4a16::rows_streams(atoi(argv[i]), atoi(argv[i + 1]), atoi(argv[i + 2]), 256));
     }
     std::printf("%d\\n", (int)(sizeof(w4a16::kRowsShapes) / sizeof(w4a16::kRowsShapes[0])));
 }
@@ -47,10 +49,22 @@ def picked(tmp_path_factory):
 
 def test_shapes_of_the_gpu_cases(picked):
     shapes, count = picked(SHAPES)
-    assert shapes == PICKED
-    assert len(set(shapes)) == count
+    assert [s[:3] for s in shapes] == PICKED
+    assert len(set(PICKED)) == count
 
 
 def test_few_rows_and_more_share_their_groups_a_step(picked):
     shapes, _ = picked([(16, 28672, 8192), (17, 28672, 8192), (11, 14344, 8192), (24, 14344, 8192)])
     assert [s[2] for s in shapes] == [4, 4, 4, 4]
+
+
+@pytest.mark.parametrize("m,n,k,streams", [
+    (2, 5120, 12288, False), (2, 5120, 17408, True), (3, 5120, 10752, True), (3, 5120, 9728, False),
+    (4, 5120, 8704, False), (4, 5120, 9728, True), (4, 9728, 8704, True),
+    (5, 4224, 5248, False), (5, 8192, 6144, False), (5, 9728, 5248, True), (5, 4224, 8192, True),
+    (6, 5120, 5248, False), (6, 5120, 6144, True), (7, 4224, 5248, True), (8, 4104, 5248, True),
+    (5, 4104, 7168, False), (4, 4104, 8704, False), (5, 4104, 8192, True), (7, 4104, 5248, False),
+    (8, 4096, 17408, False), (8, 5120, 5120, False),
+])
+def test_few_rows_route(picked, m, n, k, streams):
+    assert picked([(m, n, k)])[0][0][3] == streams

@@ -21,6 +21,11 @@ pytestmark = pytest.mark.gpu
     (8, 16648, 5248),   # five tile pairs a block
     (8, 4136, 10496),   # 82 groups: the rows no longer fit, the GEMM takes it
     (16, 4136, 5248),
+    (9, 4136, 8192),    # the longest K the LDS-staged tile-pair form holds at nine rows, and at thirteen
+    (13, 4136, 5632),
+    (10, 4136, 8192),
+    (5, 4104, 7168),    # the few-row form, two blocks of it a CU
+    (6, 4136, 5248),
 ])
 def test_linear_parity(cuda, m, n, k):
     print(f"gemm M={m} N={n} K={k}", flush=True)
