@@ -32,7 +32,8 @@
  *                       row-major rows in gemm_int4_bf16
  *   rows_stream_kernel  the down projection of up to 16 rows, more than one tile pair a CU: one
  *                       block a CU, its rows staged in LDS once, its units dealt evenly to its waves
- *   rows_gemm_kernel    M > 16, and up to 16 rows where the above give a CU too few blocks: row tiles
+ *   gemv_rows16w_kernel M > 16 with a short K and few tile pairs: the same on slices of 16 rows
+ *   rows_gemm_kernel    M > 16 otherwise, and up to 16 rows where the above give a CU too few blocks: row tiles
  *                       x tile pairs a block, the rows staged in LDS step by step
  *   mfma_gemm_kernel    2 <= M <= 16 where the above do not fit: v_mfma_f32_16x16x32_bf16, K
  *                       split across blocks
@@ -1515,6 +1516,112 @@ __device__ __forceinline__ void rows_store(float v, bool ok, int m, int tile, in
     }
 }
 
+/* More than 16 row-major rows of a K of at most 32 groups where slices of 16 rows x TPW tile pairs are no more
+ * blocks than CUs (rows_slices): gemv_rows16x_kernel's layout (16 waves a block, wave ks taking groups ks and ks + 16, each
+ * lane its own A operand from memory, one LDS meeting at the end), a wave running each A operand against TPW
+ * adjacent tile pairs. blockIdx.y takes rows 16 y .. 16 y + 15. A wave's loads are in flight at once, so a call is
+ * one round trip, where the row-tiled GEMM has one a step: 24 rows of 2560 x 1024 5.3 us, 6.1 there. */
+template <bool OUT_F32, int TPW>
+__global__ __launch_bounds__(1024) void gemv_rows16w_kernel(
+    const uint16_t *__restrict__ x, int M, const uint8_t *__restrict__ wt,
+    const uint16_t *__restrict__ st, void *__restrict__ out, int N, int K, uint16_t *residual) {
+    constexpr int SK = 16, NL = 2;
+    constexpr int D = TPW < 4 ? NL : 1; /* A groups in flight: the second beside four tile pairs costs registers */
+    __shared__ f32x4_t red[SK * TPW * 64]; /* [wave][tile pair][lane] */
+    const int G = K >> 7;
+    const int tiles = N >> 3;
+    const int lane = threadIdx.x & 63;
+    const int ks = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int q = lane >> 4, n = lane & 15, r = n & 7;
+    const int m0 = (int)blockIdx.y * 16;
+    const int rows = min(16, M - m0);
+    const int tile0 = 2 * TPW * (int)blockIdx.x + (n >> 3);
+
+    /* 1. every scale, then every weight piece of this wave (a tile past N reads zeros) */
+    const __amdgpu_buffer_rsrc_t wr = make_rsrc(wt, (uint32_t)((size_t)N * K / 2));
+    const __amdgpu_buffer_rsrc_t sr = make_rsrc(st, (uint32_t)((size_t)N * G * 2));
+    uint4 buf[NL][TPW];
+    uint16_t sbits[NL][TPW];
+#pragma unroll
+    for (int i = 0; i < NL; ++i)
+#pragma unroll
+        for (int p = 0; p < TPW; ++p) {
+            const int g = ks + i * SK, tile = tile0 + 2 * p;
+            sbits[i][p] = buf_load_u16(sr, tile < tiles && g < G ? (uint32_t)(tile * G + g) * 16 + (uint32_t)r * 2 : kOob);
+        }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < NL; ++i) {
+#pragma unroll
+        for (int p = 0; p < TPW; ++p) {
+            const int g = ks + i * SK, tile = tile0 + 2 * p;
+            buf[i][p] = buf_load16_stream(
+                wr, tile < tiles && g < G ? (uint32_t)(tile * G + g) * 512 + (uint32_t)(q * 8 + r) * 16 : kOob);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
+
+    /* 2. the A operands: for MFMA t of group i, row n, k = 128 g + 32 t + 8 q .. + 7 */
+    const __amdgpu_buffer_rsrc_t xr = make_rsrc(x + (size_t)m0 * K, (uint32_t)rows * K * 2);
+    uint4 av[D][4];
+    auto load_a = [&](int i) {
+        const int g = ks + i * SK;
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+            av[i % D][t] = buf_load16(xr, n < rows && g < G ? (uint32_t)(n * K + g * 128 + 32 * t + q * 8) * 2 : kOob);
+    };
+#pragma unroll
+    for (int i = 0; i < D; ++i) load_a(i);
+
+    /* 3. eight MFMAs a group and tile pair (the offset ones as in gemv_rows_kernel) */
+    const uint4 offs = make_uint4(0xBF40BF40u, 0xBF40BF40u, 0xBF40BF40u, 0xBF40BF40u);
+    f32x4_t acc[TPW];
+#pragma unroll
+    for (int p = 0; p < TPW; ++p) acc[p] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int i = 0; i < NL; ++i) {
+        if (ks + i * SK < G) { /* wave-uniform */
+#pragma unroll
+            for (int p = 0; p < TPW; ++p) {
+                const uint32_t words[4] = {buf[i][p].x, buf[i][p].y, buf[i][p].z, buf[i][p].w};
+                f32x4_t d = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                for (int t = 0; t < 4; ++t) {
+                    const bf16x8_t a = __builtin_bit_cast(bf16x8_t, av[i % D][t]);
+                    d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, unpack8(words[t]), d, 0, 0, 0);
+                    d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, __builtin_bit_cast(bf16x8_t, offs), d, 0, 0, 0);
+                }
+                const float sc = bf16_widen(sbits[i][p]);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) acc[p][j] = fmaf(sc, d[j], acc[p][j]);
+            }
+        } else { /* keeps the pairs' loads ahead of the branch, in issue order */
+#pragma unroll
+            for (int p = 0; p < TPW; ++p) asm volatile("" ::"v"(buf[i][p].x), "v"(sbits[i][p]));
+        }
+        if (i + D < NL) load_a(i + D);
+    }
+
+    /* 4. the 16 waves in LDS, summed in wave order; wave p finishes tile pair p */
+#pragma unroll
+    for (int p = 0; p < TPW; ++p) red[(ks * TPW + p) * 64 + lane] = acc[p];
+    __syncthreads();
+    if (ks >= TPW) return;
+    f32x4_t sum = red[ks * 64 + lane];
+    for (int w = 1; w < SK; ++w) {
+        const f32x4_t v = red[(w * TPW + ks) * 64 + lane];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) sum[j] += v[j];
+    }
+    const int tile = tile0 + 2 * ks;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const int m = 4 * q + j;
+        rows_store<OUT_F32 ? kOutF32 : kOutBf16>(32.0f * sum[j], m < rows && tile < tiles, m0 + m, tile, r, M, N, out,
+                                                 residual, 0);
+    }
+}
+
 /* A sum's rounding error grows with the length of its chains. Where a wave of rows_gemm_kernel or
  * rows_stream_kernel has more products than kFoldFrom, their FOLD forms move its accumulators into
  * second-level sums every kFold products, which keeps the error of FP32 partials at or below that of sixteen
@@ -2374,6 +2481,14 @@ int launch_rows16x(const uint16_t *x, int M, const uint8_t *w, const uint16_t *s
     return 1;
 }
 
+template <bool OUT_F32, int TPW>
+int launch_rows16w(const uint16_t *x, int M, const uint8_t *w, const uint16_t *s, void *out, int N,
+                   int K, hipStream_t stream, uint16_t *residual) {
+    launch_k((gemv_rows16w_kernel<OUT_F32, TPW>), dim3(((N / 8 + 1) / 2 + TPW - 1) / TPW, (M + 15) / 16), dim3(1024), 0,
+             stream, x, M, w, s, out, N, K, residual);
+    return hip_status(hipGetLastError(), "gemv rows16w launch");
+}
+
 template <int OUT, int MT, int TPW, int WN, int WK, bool CM = false>
 int launch_rows_gemm_cfg(const uint16_t *x, int M, const uint8_t *w, const uint16_t *s, void *out, int N,
                          int K, hipStream_t stream, uint16_t *residual, int cm) {
@@ -2419,6 +2534,21 @@ int launch_rows_gemm(const uint16_t *x, int M, const uint8_t *w, const uint16_t 
         case 11: return launch_rows_gemm_cfg<OUT, 2, 3, 2, 2>(x, M, w, s, out, N, K, stream, residual, cm);
         default: return launch_rows_gemm_cfg<OUT, 4, 2, 5, 2>(x, M, w, s, out, N, K, stream, residual, cm);
     }
+}
+
+/* More than 16 rows. */
+template <int OUT>
+int launch_many(const uint16_t *x, int M, const uint8_t *w, const uint16_t *s, void *out, int N, int K,
+                hipStream_t stream, uint16_t *residual = nullptr) {
+    if (OUT != kOutPairSilu) {
+        constexpr bool F32 = OUT == kOutF32;
+        switch (rows_slices(M, N, K, device_cus())) {
+            case 1: return launch_rows16w<F32, 1>(x, M, w, s, out, N, K, stream, residual);
+            case 2: return launch_rows16w<F32, 2>(x, M, w, s, out, N, K, stream, residual);
+            case 4: return launch_rows16w<F32, 4>(x, M, w, s, out, N, K, stream, residual);
+        }
+    }
+    return launch_rows_gemm<OUT>(x, M, w, s, out, N, K, stream, residual);
 }
 
 template <bool PAIR, bool OUT_F32>
@@ -2824,7 +2954,7 @@ static int run_rows(const uint16_t *x, int M, const uint8_t *w, const uint16_t *
                     int N, int K, hipStream_t stream, int cm = 0) {
     constexpr bool PAIR = OUT == kOutPairSilu;
     constexpr bool F32 = OUT == kOutF32;
-    if (M > 16) return launch_rows_gemm<OUT>(x, M, w, s, out, N, K, stream);
+    if (M > 16) return launch_many<OUT>(x, M, w, s, out, N, K, stream);
     /* one row: the v_dot2 GEMVs, except a pair operand past the block-staged kernel's K
      * (then the MFMA form with one live row) */
     const bool gemv = M == 1 && (!PAIR || K <= kMaxGemvK);
@@ -3131,7 +3261,7 @@ extern "C" int mlp_int4_residual_norm_bf16(uint16_t *residual, const uint16_t *s
         if (st > 0) st = launch_mfma<kOutBf16>(act, M, dnp, dns, out, hidden, inter, s, residual);
         return st;
     }
-    if (M > 16) return launch_rows_gemm<kOutBf16>(act, M, dnp, dns, out, hidden, inter, s, residual);
+    if (M > 16) return launch_many<kOutBf16>(act, M, dnp, dns, out, hidden, inter, s, residual);
     st = run_rows<kOutBf16>(act, M, dnp, dns, out, hidden, inter, s);
     if (st) return st;
     const long long chunks = (long long)M * hidden / 8;

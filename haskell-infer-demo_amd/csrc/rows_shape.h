@@ -75,6 +75,23 @@ inline bool rows_streams(int M, int N, int K, int cus) {
     return !(M >= 4 && tile_pairs < cus + cus / 32 && staged <= kMaxLds / 2);
 }
 
+/* Tile pairs a block (1, 2 or 4) of gemv_rows16w_kernel for a linear of more than 16 rows, 0 where the row-tiled
+ * GEMM takes it. The registers-fed slices win while they are one round of blocks and K is no more than two groups a
+ * wave, except where K fills the steps of the GEMM's small shapes (24 rows, N = 1024, registers-fed / row-tiled: K = 1024
+ * 4.0 / 4.3 us, 1536 4.4 / 5.4, 2048 5.0 / 4.8, 2560 5.3 / 6.1, 3712 6.1 / 6.5, 4096 6.5 / 6.5; two tile pairs, 128
+ * rows: 1024 4.5 / 4.4, 1536 5.0 / 5.4, 2560 5.9 / 6.3); in fours only as a nearly full round (K = 3200, N = 2048, 128 / 80
+ * rows 7.6 / 8.2, 7.8 / 7.5). */
+inline int rows_slices(int M, int N, int K, int cus) {
+    const int G = K / 128;
+    if ((G > 12 && G <= 16) || G > 30) return 0;
+    const long long tile_pairs = (N / 8 + 1) / 2, slices = (M + 15) / 16;
+    if (tile_pairs * slices <= cus) return 1;
+    if (G > 5 && G <= 8) return 0;
+    if ((tile_pairs + 1) / 2 * slices <= cus) return G <= 28 ? 2 : 0;
+    const long long fours = (tile_pairs + 3) / 4 * slices;
+    return fours <= cus && fours > cus * 7 / 8 ? 4 : 0;
+}
+
 }  // namespace w4a16
 
 #endif

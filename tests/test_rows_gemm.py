@@ -1,6 +1,6 @@
-"""The row-tiled GEMM (rows_gemm_kernel), where launch_rows and every call of more than 16 rows send
-work to it: each of its block shapes at the edges of their row tiles, tile pairs and K steps, against
-the oracle. The tolerances are the suite's (assert_parity): 2 BF16 ULP and rel-L2 1e-3 of the double-accumulated
+"""The row-tiled GEMM (rows_gemm_kernel), where launch_rows and calls of more than 16 rows send work to
+it: each of its block shapes at the edges of their row tiles, tile pairs and K steps, against the oracle;
+and the slices of 16 rows (gemv_rows16w_kernel) that some of the latter run as. The tolerances are the suite's (assert_parity): 2 BF16 ULP and rel-L2 1e-3 of the double-accumulated
 product."""
 
 import numpy as np
@@ -16,23 +16,33 @@ pytestmark = pytest.mark.gpu
 
 # (rows, N, K): one half-filled tile pair of one group; then every block shape (row tiles x tile
 # pairs x groups a step) where the launcher's estimate picks it, with odd tile counts, rows that do
-# not fill the row tiles and K that does not fill the steps
+# not fill the row tiles and K that does not fill the steps; the slices of 16 rows by one, two and four tile
+# pairs a block likewise
 SHAPES = [
-    (17, 8, 128),        # 1 x 4 x 4
+    (17, 8, 128),        # slices, one tile pair
     (17, 8, 5248),       # 1 x 1 x 16
     (16, 520, 9856),     # 1 x 1 x 16, past the tile-pair form
-    (17, 8, 640),        # 1 x 2 x 8
-    (33, 2568, 2688),    # 1 x 3 x 8
+    (17, 8, 640),        # slices, one tile pair
+    (17, 8, 2048),       # 1 x 2 x 8
+    (33, 2568, 2688),    # slices, two tile pairs
+    (33, 2568, 3712),    # 1 x 3 x 8
     (33, 2568, 1664),    # 1 x 4 x 4
-    (33, 5128, 640),     # 1 x 6 x 4
+    (33, 5128, 640),     # slices, four tile pairs
+    (33, 5640, 640),     # 1 x 6 x 4
     (33, 9736, 1152),    # 1 x 8 x 4
-    (33, 5128, 128),     # 1 x 10 x 2
+    (33, 5128, 128),     # slices, four tile pairs
+    (33, 5640, 128),     # 1 x 10 x 2
     (17, 12296, 640),    # 2 x 4 x 4
     (120, 5128, 1152),   # 2 x 6 x 4
     (50, 12296, 2688),   # 2 x 9 x 4
     (63, 19464, 640),    # 2 x 10 x 2
     (120, 5128, 640),    # 2 x 6 x 2
     (127, 19464, 640),   # 4 x 10 x 2
+    (50, 1000, 3840),    # slices, one tile pair, two groups a wave but for two of them
+    (40, 1032, 1536),    # slices, one tile pair, twelve of sixteen waves
+    (97, 1032, 2176),    # slices, two tile pairs
+    (127, 2040, 3200),   # slices, four tile pairs
+    (255, 1016, 1280),   # slices, four tile pairs
 ]
 
 

@@ -19,16 +19,17 @@ MAIN = """
 int main(int argc, char **argv) {
     for (int i = 1; i + 2 < argc; i += 3) {
         const auto &s = w4a16::kRowsShapes[w4a16::rows_shape(atoi(argv[i]), atoi(argv[i + 1]), atoi(argv[i + 2]), 256)];
-        std::printf("%d %d %d %d\\n", s.rows, s.tile_pairs, s.groups,
-                    (int)w4a16::rows_streams(atoi(argv[i]), atoi(argv[i + 1]), atoi(argv[i + 2]), 256));
+        std::printf("%d %d %d %d %d\\n", s.rows, s.tile_pairs, s.groups,
+                    (int)w4a16::rows_streams(atoi(argv[i]), atoi(argv[i + 1]), atoi(argv[i + 2]), 256),
+                    w4a16::rows_slices(atoi(argv[i]), atoi(argv[i + 1]), atoi(argv[i + 2]), 256));
     }
     std::printf("%d\\n", (int)(sizeof(w4a16::kRowsShapes) / sizeof(w4a16::kRowsShapes[0])));
 }
 """
 
-# row tiles x tile pairs x groups a step of each of SHAPES
-PICKED = [(1, 4, 4), (1, 1, 16), (1, 1, 16), (1, 2, 8), (1, 3, 8), (1, 4, 4), (1, 6, 4), (1, 8, 4), (1, 10, 2),
-          (2, 4, 4), (2, 6, 4), (2, 9, 4), (2, 10, 2), (2, 6, 2), (4, 10, 2)]
+# row tiles x tile pairs x groups a step of each of SHAPES, or the tile pairs of its slices of 16 rows
+PICKED = [1, (1, 1, 16), (1, 1, 16), 1, (1, 2, 8), 2, (1, 3, 8), (1, 4, 4), 4, (1, 6, 4), (1, 8, 4),
+          4, (1, 10, 2), (2, 4, 4), (2, 6, 4), (2, 9, 4), (2, 10, 2), (2, 6, 2), (4, 10, 2), 1, 1, 2, 4, 4]
 
 
 @pytest.fixture(scope="module")
@@ -49,8 +50,8 @@ def picked(tmp_path_factory):
 
 def test_shapes_of_the_gpu_cases(picked):
     shapes, count = picked(SHAPES)
-    assert [s[:3] for s in shapes] == PICKED
-    assert len(set(PICKED)) == count
+    assert [m > 16 and s[4] or s[:3] for (m, _, _), s in zip(SHAPES, shapes)] == PICKED
+    assert len({p for p in PICKED if not isinstance(p, int)}) == count
 
 
 def test_few_rows_and_more_share_their_groups_a_step(picked):
@@ -68,3 +69,13 @@ def test_few_rows_and_more_share_their_groups_a_step(picked):
 ])
 def test_few_rows_route(picked, m, n, k, streams):
     assert picked([(m, n, k)])[0][0][3] == streams
+
+
+@pytest.mark.parametrize("m,n,k,tile_pairs", [
+    (24, 1024, 1024, 1), (24, 1024, 1536, 1), (24, 1024, 1664, 0), (24, 1024, 2048, 0), (24, 1024, 2560, 1),
+    (24, 1024, 3840, 1), (24, 1024, 3968, 0), (64, 1024, 2560, 1), (65, 1024, 2560, 2), (128, 1024, 2560, 2),
+    (128, 1024, 1024, 0), (128, 1024, 640, 2), (24, 2560, 3712, 0), (128, 2048, 3200, 4), (80, 2048, 3200, 0),
+    (128, 4096, 2560, 0), (128, 128, 128, 1), (100000, 128, 128, 0),
+])
+def test_slices_route(picked, m, n, k, tile_pairs):
+    assert picked([(m, n, k)])[0][0][4] == tile_pairs
