@@ -1993,8 +1993,8 @@ __global__ __launch_bounds__(1024) void rows_stream_kernel(
  * 8-value chunks of the row, all loaded before any use, so a row costs one load round trip;
  * cols % 8 == 0 and cols <= CH * 8 * blockDim.x <= 16384 (the launcher checks).
  *
- * What bounds it is latency: launch, one round trip, the chain of FP64 sums and the scale. As many
- * threads as chunks (up to 1024) keep a thread's part of the chain to eight sums; 16 x 5120
+ * What bounds it for few rows is latency: launch, one round trip, the chain of FP64 sums and the scale. As many
+ * threads as chunks (up to 1024; half of that where many rows share a CU, rmsnorm_chunks) keep a thread's part of the chain to eight sums; 16 x 5120
  * repeated in a graph 2.51 -> 2.26 us, 4 x 2560 2.23 -> 2.10, with norm_scale and wave_sum_f64 (2.0 of it
  * is a launch that depends on the one before). */
 template <int CH>
@@ -3106,7 +3106,7 @@ static int launch_rmsnorm(uint16_t *out, const uint16_t *x, const uint16_t *w, i
     if (cols % 8 || chunks > 2048)
         return set_error(W4A16_ERR_CONFIG, "rmsnorm: cols=%d must be a multiple of 8 and <= 16384",
                          cols);
-    const int ch = chunks > 1024 ? 2 : 1;
+    const int ch = rmsnorm_chunks(cols, rows, device_cus());
     const dim3 block((chunks + 64 * ch - 1) / (64 * ch) * 64);
     if (ch == 1)
         launch_k(rmsnorm_kernel<1>, dim3(rows), block, 0, s, out, const_cast<uint16_t *>(x), w, cols, bias, eps, 1.0 / cols, sub);

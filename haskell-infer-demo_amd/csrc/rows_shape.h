@@ -1,6 +1,6 @@
 /*
  * rows_shape.h - host-only rules of the multi-row dispatch: the block shapes of rows_gemm_kernel and the choice
- * between them, and which linears of a few rows rows_stream_kernel takes.
+ * between them, which linears rows_stream_kernel and gemv_rows16w_kernel take, and the RMSNorm's block.
  */
 #ifndef W4A16_ROWS_SHAPE_H
 #define W4A16_ROWS_SHAPE_H
@@ -90,6 +90,14 @@ inline int rows_slices(int M, int N, int K, int cus) {
     if ((tile_pairs + 1) / 2 * slices <= cus) return G <= 28 ? 2 : 0;
     const long long fours = (tile_pairs + 3) / 4 * slices;
     return fours <= cus && fours > cus * 7 / 8 ? 4 : 0;
+}
+
+/* Chunks of 8 values a thread of rmsnorm_kernel. One keeps a row's FP64 chain shortest; of blocks past 512 threads,
+ * though, too few fit a CU once there are more rows than that (5120 columns, one / two chunks: 384 rows and fewer one is
+ * ahead, 768 4.7 / 4.2 us, 2048 8.7 / 7.9, 16384 69 / 58). */
+inline int rmsnorm_chunks(int cols, int rows, int cus) {
+    const int chunks = cols / 8;
+    return chunks > 1024 || (chunks > 512 && rows > cus + cus / 2) ? 2 : 1;
 }
 
 }  // namespace w4a16

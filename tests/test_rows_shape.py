@@ -1,5 +1,5 @@
 """The host-only rules of the multi-row dispatch on 256 CUs: the block shapes of the row-tiled GEMM's GPU cases are
-the ones the launcher picks, with all shapes among them, and the linears of a few rows go to the kernel that
+the ones the launcher picks, with all shapes among them, and linears and norms go to the kernel or block that
 measured faster. rows_shape.h is compiled here as it stands."""
 
 import os
@@ -19,9 +19,10 @@ MAIN = """
 int main(int argc, char **argv) {
     for (int i = 1; i + 2 < argc; i += 3) {
         const auto &s = w4a16::kRowsShapes[w4a16::rows_shape(atoi(argv[i]), atoi(argv[i + 1]), atoi(argv[i + 2]), 256)];
-        std::printf("%d %d %d %d %d\\n", s.rows, s.tile_pairs, s.groups,
+        std::printf("%d %d %d %d %d %d\\n", s.rows, s.tile_pairs, s.groups,
                     (int)w4a16::rows_streams(atoi(argv[i]), atoi(argv[i + 1]), atoi(argv[i + 2]), 256),
-                    w4a16::rows_slices(atoi(argv[i]), atoi(argv[i + 1]), atoi(argv[i + 2]), 256));
+                    w4a16::rows_slices(atoi(argv[i]), atoi(argv[i + 1]), atoi(argv[i + 2]), 256),
+                    w4a16::rmsnorm_chunks(atoi(argv[i + 1]), atoi(argv[i]), 256));
     }
     std::printf("%d\\n", (int)(sizeof(w4a16::kRowsShapes) / sizeof(w4a16::kRowsShapes[0])));
 }
@@ -79,3 +80,10 @@ def test_few_rows_route(picked, m, n, k, streams):
 ])
 def test_slices_route(picked, m, n, k, tile_pairs):
     assert picked([(m, n, k)])[0][0][4] == tile_pairs
+
+
+@pytest.mark.parametrize("rows,cols,chunks", [
+    (1, 5120, 1), (384, 5120, 1), (385, 5120, 2), (16384, 4096, 1), (16384, 4104, 2), (385, 8192, 2), (1, 8200, 2),
+])
+def test_rmsnorm_block(picked, rows, cols, chunks):
+    assert picked([(rows, cols, 128)])[0][0][5] == chunks
