@@ -200,8 +200,9 @@ def _stream(stream):
     if stream is None:
         import torch
 
-        # the handle itself: building the Stream object around it takes longer than a kernel's launch
-        return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
+        # the handle itself where torch gives it: building the Stream object around it takes longer than a launch
+        raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+        return torch.cuda.current_stream().cuda_stream if raw is None else raw(torch.cuda.current_device())
     if isinstance(stream, int):
         return stream
     return stream.cuda_stream
