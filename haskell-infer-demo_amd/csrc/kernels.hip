@@ -24,18 +24,20 @@
  *                       gate/up pair
  *   gemv_rows_kernel    2 <= M <= 8: the GEMV's block structure on v_mfma_f32_16x16x32_bf16 with
  *                       a block-diagonal operand, activation loaded straight into LDS
- *   gemv_rows16_kernel  9 <= M <= 16, short K: the same with a tile pair a wave
+ *   gemv_rows16_kernel  9 <= M <= 16, the rows fitting LDS: the same with a tile pair a wave
  *   gemv_rows16x_kernel long K, no pair (the down projection): a tile pair a block, each lane
  *                       loading its MFMA A operand from memory into registers (no LDS staging,
- *                       no K split across blocks); 4 <= M <= 16 inside the FFN entry points,
- *                       which keep the intermediate chunk-major for it, 8 <= M <= 15 on
- *                       row-major rows in gemm_int4_bf16
- *   rows_stream_kernel  the down projection of up to 16 rows, more than one tile pair a CU: one
- *                       block a CU, its rows staged in LDS once, its units dealt evenly to its waves
+ *                       no K split across blocks), up to one tile pair a CU; 4 <= M <= 16 inside the
+ *                       FFN entry points, which keep the intermediate chunk-major for it, 8 <= M <= 15
+ *                       on row-major rows
+ *   rows_stream_kernel  long K, no pair, up to 16 rows, more than one tile pair a CU: blocks of an equal
+ *                       share of tile pairs, at most one a CU, the rows staged in LDS once and the
+ *                       share's units dealt evenly to the waves
  *   gemv_rows16w_kernel M > 16 with a short K and few tile pairs: the same on slices of 16 rows
  *   rows_gemm_kernel    M > 16 otherwise, and up to 16 rows where the above give a CU too few blocks: row tiles
  *                       x tile pairs a block, the rows staged in LDS step by step
- *   mfma_gemm_kernel    2 <= M <= 16 where the above do not fit: v_mfma_f32_16x16x32_bf16, K
+ *   mfma_gemm_kernel    up to 8 rows where the above do not fit (the pair at one row past the GEMV's
+ *                       K, few rows whose staged copies exceed LDS): v_mfma_f32_16x16x32_bf16, K
  *                       split across blocks
  *   rmsnorm_kernel, residual_add_kernel, silu_mul_packed_kernel: the norm, the residual update
  *                       and the standalone SiLU x up
@@ -1225,7 +1227,7 @@ __global__ __launch_bounds__(TB * SK * 64) void gemv_rows_kernel(
     }
 }
 
-/* Up to 16 rows (9 <= M <= 16), short K: as gemv_rows_kernel, but a wave owns a tile pair and a
+/* Up to 16 rows (9 <= M <= 16) that fit LDS: as gemv_rows_kernel, but a wave owns a tile pair and a
  * load covers one group of both tiles (lane l: piece (row l & 7, kb = l >> 4) of tile
  * 2 tp + ((l >> 3) & 1)), so all sixteen B columns share the k range and all sixteen A rows are
  * activation rows. A block holds blockDim / 64 waves: TP tile pairs of SK waves (both runtime),
@@ -1832,7 +1834,8 @@ __global__ __launch_bounds__(WN * WK * 64) void rows_gemm_kernel(
 }
 
 /* The down projection of a few rows (K x rows up to 160 KB of LDS) with more than one tile pair a
- * CU: one block of 16 waves a CU owns TPB <= 16 tile pairs over all of K and stages its rows in LDS
+ * CU: a block of 16 waves owns TPB <= 16 tile pairs over all of K, TPB the least that makes no more blocks
+ * than CUs (5120 outputs: 2 and 160 blocks; 4224: 132; 8192: 256), and stages its rows in LDS
  * once (chunk c of row m in slot c ^ m or, with CM, as the chunk-major activation lies in memory).
  * The block's TPB x G units (a group of a tile pair, 1 KiB of weight) are then dealt to its waves in
  * equal contiguous ranges, tile pair by tile pair, so no wave idles where TPB is no multiple of
@@ -2470,8 +2473,8 @@ template <bool OUT_F32, bool CM = false>
 int launch_rows16x(const uint16_t *x, int M, const uint8_t *w, const uint16_t *s, void *out, int N,
                    int K, hipStream_t stream, uint16_t *residual = nullptr) {
     const int nl = (K / 128 + 15) / 16;
-    if (nl <= 2) return launch_rows16x_nl<OUT_F32, CM, 2>(x, M, w, s, out, N, K, stream, residual);
-    if (nl <= 3) return launch_rows16x_nl<OUT_F32, CM, 3>(x, M, w, s, out, N, K, stream, residual);
+    if constexpr (!CM) /* row-major from 39 groups (launch_rows), chunk-major from 64 */
+        if (nl <= 3) return launch_rows16x_nl<OUT_F32, CM, 3>(x, M, w, s, out, N, K, stream, residual);
     if (nl <= 4) return launch_rows16x_nl<OUT_F32, CM, 4>(x, M, w, s, out, N, K, stream, residual);
     if (nl <= 5) return launch_rows16x_nl<OUT_F32, CM, 5>(x, M, w, s, out, N, K, stream, residual);
     if (nl <= 6) return launch_rows16x_nl<OUT_F32, CM, 6>(x, M, w, s, out, N, K, stream, residual);
@@ -2785,7 +2788,7 @@ MfmaPlan plan_mfma(int M, int N, int K) {
     p.S = (G + p.GS - 1) / p.GS;
     const int chunks = M * p.GS * 16;
     const int pre = (chunks + kMfmaWaves * 64 - 1) / (kMfmaWaves * 64);
-    p.xpre = pre <= 1 ? 1 : pre <= 2 ? 2 : pre <= 4 ? 4 : 8;
+    p.xpre = pre <= 1 ? 1 : pre <= 2 ? 2 : 4; /* at most 8 rows of kGMax groups: 4 */
     p.grid = nblk * p.S;
     p.smem = (size_t)(chunks + p.GS * 16) * 16 + (size_t)M * p.GS * 4;
     p.partial_bytes = p.S > 1 ? (size_t)p.S * NT * 16 * M * sizeof(uint64_t) : 0;
@@ -2844,7 +2847,9 @@ int fixed_scratch(hipStream_t stream, unsigned char **base) {
 
 /* An upper bound of the split-K scratch one [M, K] x [N, K]^T product of this library can ask
  * for, whichever kernel it is routed to: the wave-local GEMV's tile split (at most 8 blocks a
- * tile, M = 1) and the MFMA form's plan for a 16-row slice (smaller slices need less). */
+ * tile, M = 1) and the MFMA form's plan (M <= 8). No kernel of more rows takes any; the plan of up
+ * to 16 rows stands in the limit of mlp_int4_bf16_noalloc, which is on sizes alone and refuses what it
+ * always has. */
 void split_bound(int M, int N, int K, size_t *partial_bytes, size_t *ncounters) {
     const size_t tiles = (size_t)N / 8;
     size_t pb = tiles * 8 * 8 * sizeof(uint64_t), nc = tiles;
@@ -2874,7 +2879,7 @@ int launch_mfma_x(const MfmaPlan &p, const uint16_t *x, int M, const uint8_t *w,
     return hip_status(hipGetLastError(), "mfma gemm launch");
 }
 
-/* M <= 16 rows of x against a tile-order weight. */
+/* M <= 8 rows of x against a tile-order weight. */
 template <int OUT>
 int launch_mfma(const uint16_t *x, int M, const uint8_t *w, const uint16_t *s, void *out, int N,
                 int K, hipStream_t stream, uint16_t *residual = nullptr, int cm = 0) {
@@ -2888,8 +2893,7 @@ int launch_mfma(const uint16_t *x, int M, const uint8_t *w, const uint16_t *s, v
     switch (p.xpre) {
         case 1: return launch_mfma_x<OUT, 1>(p, x, M, w, s, out, N, K, partial, counters, stream, residual, cm);
         case 2: return launch_mfma_x<OUT, 2>(p, x, M, w, s, out, N, K, partial, counters, stream, residual, cm);
-        case 4: return launch_mfma_x<OUT, 4>(p, x, M, w, s, out, N, K, partial, counters, stream, residual, cm);
-        default: return launch_mfma_x<OUT, 8>(p, x, M, w, s, out, N, K, partial, counters, stream, residual, cm);
+        default: return launch_mfma_x<OUT, 4>(p, x, M, w, s, out, N, K, partial, counters, stream, residual, cm);
     }
 }
 
@@ -2948,7 +2952,7 @@ int check_gemm_args(const void *a, const void *p, const void *s, const void *o, 
 /* ---------------------------------------------------------------------------------------- */
 
 /* Rows of x: M = 1 takes the v_dot2 GEMV; 2 <= M <= 16 the kernels of launch_rows, or the split-K
- * MFMA form where they have no shape; larger M the row-tiled GEMM. */
+ * MFMA form where they have no shape; larger M those of launch_many. */
 template <int OUT>
 static int run_rows(const uint16_t *x, int M, const uint8_t *w, const uint16_t *s, void *out,
                     int N, int K, hipStream_t stream, int cm = 0) {
@@ -3027,11 +3031,11 @@ extern "C" int mlp_int4_bf16(const uint16_t *normed, const uint8_t *gup, const u
 }
 
 /* Grows the per-device split-K scratch (current device) to the worst case of every FFN call of
- * 1..max_rows rows at this shape, so that such calls never allocate afterwards. The loader calls
+ * 1..max_rows rows at this shape (calls of more than 8 use none), so that such calls never allocate afterwards. The loader calls
  * it once per store, outside any capture. */
 int reserve_split_scratch(int max_rows, int hidden, int inter) {
     size_t pb = 0, nc = 0;
-    for (int m = 1; m <= std::max(1, std::min(max_rows, 16)); ++m) {
+    for (int m = 1; m <= std::max(1, std::min(max_rows, 8)); ++m) {
         size_t a, b, c, d;
         split_bound(m, 2 * inter, hidden, &a, &b);
         split_bound(m, hidden, inter, &c, &d);

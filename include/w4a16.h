@@ -151,7 +151,8 @@ int mlp_int4_bf16(const uint16_t *normed, const uint8_t *gu_packed, const uint16
  * array of the library (256 KiB of counters and 32 MiB of partial slots a GPU, held until the
  * process ends) instead of the growable per-device buffer, so no call allocates or
  * synchronises. Shapes whose worst-case split-K need exceeds that array are refused with
- * W4A16_ERR_CONFIG before anything is launched (every BASELINE shape up to M = 16 fits). The
+ * W4A16_ERR_CONFIG before anything is launched, with M up to 16 counted as if it took the split-K
+ * form, which runs up to 8 rows (hidden 5120, intermediate 17408 fits at any M). The
  * first call on a device looks the array up and clears the array with a kernel on `stream`.
  * Every call on one GPU shares the array: calls that overlap in time on one GPU race, so order
  * them on one stream. */
