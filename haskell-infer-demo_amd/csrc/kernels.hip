@@ -1625,14 +1625,14 @@ __global__ __launch_bounds__(1024) void gemv_rows16w_kernel(
 }
 
 /* A sum's rounding error grows with the length of its chains. Where a wave of rows_gemm_kernel or
- * rows_stream_kernel has more products than kFoldFrom, their FOLD forms move its accumulators into
- * second-level sums every kFold products, which keeps the error of FP32 partials at or below that of sixteen
- * accumulators a column (17408 x 5120 against 64 bits, relative 2-norm, 33 / 128 / 200 rows: sixteen accumulators
- * 1.68e-7 / 1.68e-7 / 1.67e-7, chains of 34, 34 and 68 1.80e-7 / 1.79e-7 / 2.04e-7). Up to 8 row-major rows
- * the shorter chains of gemv_rows_kernel are the measure, with kFoldFew (2 rows 1.61e-7 there, in chains of
- * 17 1.66e-7, here 1.59e-7). The gate/up pair, which ends in BF16, keeps up to kFoldFromPair: folding costs a block the
- * LDS that lets the next one start (5120 x 34816 at 128 rows 97 -> 104 us). */
-constexpr int kFold = 16, kFoldFrom = 17, kFoldFew = 6, kFoldFromPair = 20;
+ * rows_stream_kernel has more products than kFoldFrom (kFoldFromTwo with two waves over K), their FOLD forms move its
+ * accumulators into second-level sums every kFold products, which keeps the error of FP32 partials at or below that
+ * of sixteen accumulators a column (17408 x 5120 against 64 bits, relative 2-norm, 33 / 128 / 200 rows: sixteen
+ * accumulators 1.68e-7 / 1.68e-7 / 1.67e-7, chains of 34, 34 and 68 1.80e-7 / 1.79e-7 / 2.04e-7, folded 1.66e-7 /
+ * 1.66e-7 / 1.65e-7; 5120 x 5120 at 200 rows, chains of 20, 1.63e-7 either way). Up to 8 row-major rows the shorter
+ * chains of gemv_rows_kernel are the measure, with kFoldFew (2 rows 1.61e-7 there, in chains of 17 1.66e-7, folded
+ * 1.59e-7). */
+constexpr int kFold = 16, kFoldFrom = 17, kFoldFromTwo = 20, kFoldFew = 6;
 
 /* Rows by tiles of 16: a block of WN x WK waves owns WN * TPW tile pairs and 16 MT activation rows
  * over all of K. In each step wave (wn, wk) takes group c WK + wk of its TPW tile pairs from memory
@@ -1917,7 +1917,7 @@ __global__ __launch_bounds__(1024) void rows_stream_kernel(
 
     const uint4 offs = make_uint4(0xBF40BF40u, 0xBF40BF40u, 0xBF40BF40u, 0xBF40BF40u);
     f32x4_t acc = {0.0f, 0.0f, 0.0f, 0.0f}, first = acc, folded = acc;
-    int since = 0; /* units in acc */
+    int since = 0; /* units since the last fold */
     const int arow = min(n, M - 1);
     int cu = u0, cg = u0 - p0 * G;
     const int cnt = u1 - u0;
@@ -1939,18 +1939,12 @@ __global__ __launch_bounds__(1024) void rows_stream_kernel(
 #pragma unroll
                 for (int j = 0; j < 4; ++j) acc[j] = fmaf(sc, d[j], acc[j]);
                 ++cu;
-                if (FOLD && ++since == kFoldFew) {
-                    since = 0;
-                    folded += acc;
-                    acc = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-                }
                 if (++cg == G) { /* the end of a tile pair: the wave's range may go on into the next */
                     cg = 0;
                     if (cu < u1) {
                         first = acc;
                         acc = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
                         if (FOLD) {
-                            since = 0;
                             first += folded;
                             folded = acc;
                         }
@@ -1958,6 +1952,11 @@ __global__ __launch_bounds__(1024) void rows_stream_kernel(
                 }
             }
             load_w(b);
+        }
+        if (FOLD && (since += PD) == kFoldFew) {
+            since = 0;
+            folded += acc;
+            acc = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
         }
     }
     __syncthreads();
@@ -2499,7 +2498,7 @@ int launch_rows_gemm_cfg(const uint16_t *x, int M, const uint8_t *w, const uint1
     static_assert(stage + reduce <= kMaxLds, "the two staged steps and the reduction fit a block's LDS");
     const bool few = M <= 8 && !CM;
     const int period = few ? kFoldFew : kFold;
-    const bool fold = K / 128 > (few ? kFoldFew : OUT == kOutPairSilu ? kFoldFromPair : kFoldFrom) * WK;
+    const bool fold = K / 128 > (few ? kFoldFew : WK == 2 ? kFoldFromTwo : kFoldFrom) * WK;
     const size_t smem = fold ? stage + reduce : std::max(stage, reduce);
     constexpr size_t elem = OUT == kOutF32 ? 4 : 2;
     const int cols = (((N / 8 + 1) / 2 + WN * TPW - 1) / (WN * TPW) + 7) / 8 * 8;
