@@ -1655,8 +1655,8 @@ constexpr int kFold = 16, kFoldFrom = 17, kFoldFromTwo = 20, kFoldFew = 6;
  * 34816 the weight stream alone in this block shape takes 19 of 23 us.
  * Whole calls, on the kernels before / here: gate/up 2560 x 19456 M = 32 / 64 / 128 18.1 / 35.3 / 68.9 ->
  * 12.8 / 18.0 / 28.9 us; 5120 x 34816 M = 16 / 32 / 64 / 128 61 / 120 / 241 / 480 -> 23.5 / 29.7 / 49 / 97;
- * down 9728 x 2560 M = 32 / 64 / 128 24.2 / 35.9 / 57.4 -> 12.5 / 14.3 / 22.3; 17408 x 5120 M = 16 /
- * 32 / 64 / 128 24.8 / 61 / 100 / 194 -> 20.6 / 23.7 / 34.9 / 50.2. */
+ * down 9728 x 2560 M = 32 / 64 / 128 24.2 / 35.9 / 57.4 -> 12.5 / 14.1 / 22.2; 17408 x 5120 M = 32 / 64 / 128
+ * 62 / 102 / 200 -> 23.9 / 36.3 / 53.8 (35.5 and 51.6 without second-level sums). */
 template <int OUT, int MT, int TPW, int WN, int WK, bool CM, bool FOLD>
 __global__ __launch_bounds__(WN * WK * 64) void rows_gemm_kernel(
     const uint16_t *__restrict__ x, int M, const uint8_t *__restrict__ wt,

@@ -131,8 +131,8 @@ def test_gemv_parity(cuda, n, k):
 
 @pytest.mark.parametrize("m", [3, 5, 7, 13, 17, 40])
 def test_small_m_parity(cuda, m):
-    """The MFMA form at row counts between the instantiated ones (3, 5, 7, 13 take the 4-row
-    and 16-row A layouts with zero rows) and past 16 (17 and 40 run 16-row slices)."""
+    """Row counts between the instantiated ones: 3, 5 and 7 on the few-row form, 13 on the LDS-staged
+    tile-pair form with zero rows, 17 and 40 in slices of 16 rows by two tile pairs."""
     n, k = 2560, 3200  # odd group count: the last group pair is half empty
     say(f"gemm M={m} n={n} k={k}")
     p, s = make_weight(n, k, seed=77)
@@ -146,11 +146,9 @@ def test_small_m_parity(cuda, m):
                                  (100, 512), (100, 4096), (128, 1024)])
 def test_m_sweep_parity(cuda, m, n):
     """The reference's --time sweep shape (K = 5120; reference tests/test_quantization_kernel.py:
-    162-216 times M = 1..128 at N = 4096): at 16 rows the registers-fed long-K kernel (the staged
-    rows would not fit LDS), past 16 all the 16-row slices in one launch, on the kernel that runs
-    each A operand against two tile pairs (32 rows at N = 4096, 128 rows at N = 1024) or four
-    (64 and 100 rows at N = 4096) where that still leaves a block a CU, else one; a ragged last
-    slice at 40 and 100 rows."""
+    162-216 times M = 1..128 at N = 4096), from 16 rows on the row-tiled GEMM: one row tile a block at
+    N = 512 and 1024 and up to 64 rows at N = 4096, two at 100 rows there; a ragged last row tile at
+    40 and 100 rows."""
     k = 5120
     say(f"gemm M={m} n={n} k={k}")
     p, s = make_weight(n, k, seed=500 + m)
@@ -198,7 +196,7 @@ def test_few_rows_parity(cuda, m):
 
 def test_random_shapes_parity(cuda):
     """Seeded random shapes across the routing boundaries (group-pair counts from 1 to 40, the
-    staged-row LDS limits, M from 1 to 20 including the 16-row slicing), through gemm_int4_bf16
+    staged-row LDS limits, M from 1 to 20 on both sides of 16), through gemm_int4_bf16
     and the fused gate/up, each against the oracle."""
     rng = np.random.default_rng(2026)
     for case in range(40):

@@ -4,10 +4,9 @@ Its split-K partials and counters live in the library's static device array inst
 growable per-device buffer; the kernels are the same, so its output must equal mlp_int4_bf16's
 bit for bit (the split-K combines sum in a fixed order). Checked on calls in a row whose second
 input is smaller, on the two routes that use the scratch: the M = 1 down projection split over
-three blocks a tile (K = 17408, then K = 13312), config 2 at 16 rows (its gate/up pair on the
-split-K MFMA form: the largest partials the bound admits among the BASELINE shapes) and the
-16-row split-K MFMA down projection (K = 25600, then 9 rows at K = 17408); then the call
-captured into a HIP graph, replayed with eager calls between the replays. Shapes beyond the
+three blocks a tile (K = 17408, then K = 13312) and the split-K MFMA down projection of a few rows
+(6, then 3 at K = 25600); on calls of 9 and 16 rows, which take none though their sizes count
+towards the limit; then the call captured into a HIP graph, replayed with eager calls between the replays. Shapes beyond the
 array are refused before any launch, and a first call on a device made under graph capture is
 refused (it would only record the one-time clear), in a fresh process.
 """
@@ -53,7 +52,7 @@ def call(fn, torch, x, gu, dn, M, hidden, inter):
 
 # (M, hidden, inter): each second case is the smaller input of its pair
 CASES = [(1, 5120, 17408), (1, 2048, 13312), (16, 5120, 17408), (16, 1024, 25600),
-         (9, 1024, 17408)]
+         (9, 1024, 17408), (6, 1024, 25600), (3, 512, 25600)]
 
 
 def test_noalloc_matches_mlp_int4(cuda):
