@@ -1995,10 +1995,10 @@ __global__ __launch_bounds__(1024) void rows_stream_kernel(
  * 8-value chunks of the row, all loaded before any use, so a row costs one load round trip;
  * cols % 8 == 0 and cols <= CH * 8 * blockDim.x <= 16384 (the launcher checks).
  *
- * What bounds it for few rows is latency: launch, one round trip, the chain of FP64 sums and the scale. As many
- * threads as chunks (up to 1024; half of that where many rows share a CU, rmsnorm_chunks) keep a thread's part of the chain to eight sums; 16 x 5120
- * repeated in a graph 2.51 -> 2.26 us, 4 x 2560 2.23 -> 2.10, with norm_scale and wave_sum_f64 (2.0 of it
- * is a launch that depends on the one before). */
+ * What bounds it for few rows is latency: launch, one round trip, the chain of FP64 sums and the scale.
+ * As many threads as chunks (up to 1024; half of that where many rows share a CU, rmsnorm_chunks) keep a
+ * thread's part of the chain to eight sums; 16 x 5120 repeated in a graph 2.51 -> 2.26 us, 4 x 2560 2.23 ->
+ * 2.10, with norm_scale and wave_sum_f64 (2.0 of it is a launch that depends on the one before). */
 template <int CH>
 __global__ __launch_bounds__(1024) void rmsnorm_kernel(uint16_t *__restrict__ out, uint16_t *x,
                                                        const uint16_t *__restrict__ w, int cols,

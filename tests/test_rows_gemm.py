@@ -1,7 +1,7 @@
 """The row-tiled GEMM (rows_gemm_kernel), where launch_rows and calls of more than 16 rows send work to
 it: each of its block shapes at the edges of their row tiles, tile pairs and K steps, against the oracle;
-and the slices of 16 rows (gemv_rows16w_kernel) that some of the latter run as. The tolerances are the suite's (assert_parity): 2 BF16 ULP and rel-L2 1e-3 of the double-accumulated
-product."""
+and the slices of 16 rows (gemv_rows16w_kernel) that some of the latter run as. The tolerances are the
+suite's (assert_parity): 2 BF16 ULP and rel-L2 1e-3 of the double-accumulated product."""
 
 import numpy as np
 import pytest
