@@ -1630,9 +1630,9 @@ __global__ __launch_bounds__(1024) void gemv_rows16w_kernel(
  * of sixteen accumulators a column (17408 x 5120 against 64 bits, relative 2-norm, 33 / 128 / 200 rows: sixteen
  * accumulators 1.68e-7 / 1.68e-7 / 1.67e-7, chains of 34, 34 and 68 1.80e-7 / 1.79e-7 / 2.04e-7, folded 1.66e-7 /
  * 1.66e-7 / 1.65e-7; 5120 x 5120 at 200 rows, chains of 20, 1.63e-7 either way). Up to 8 row-major rows the shorter
- * chains of gemv_rows_kernel are the measure, with kFoldFew (2 rows 1.61e-7 there, in chains of 17 1.66e-7, folded
- * 1.59e-7). */
-constexpr int kFold = 16, kFoldFrom = 17, kFoldFromTwo = 20, kFoldFew = 6;
+ * chains of gemv_rows_kernel are the measure, with kFoldFew from kFoldFewFrom (2 rows of 17408 x 5120 1.0358 of its
+ * error in chains of 17, 0.998 folded; 5 of 8064 x 5120 1.009 in chains of 8, 0.998 folded, and in sixes 1.005). */
+constexpr int kFold = 16, kFoldFrom = 17, kFoldFromTwo = 20, kFoldFew = 4, kFoldFewFrom = 6;
 
 /* Rows by tiles of 16: a block of WN x WK waves owns WN * TPW tile pairs and 16 MT activation rows
  * over all of K. In each step wave (wn, wk) takes group c WK + wk of its TPW tile pairs from memory
@@ -2496,9 +2496,9 @@ int launch_rows_gemm_cfg(const uint16_t *x, int M, const uint8_t *w, const uint1
                          int K, hipStream_t stream, uint16_t *residual, int cm) {
     constexpr size_t stage = (size_t)2 * WK * 16 * MT * 256, reduce = (size_t)WK * WN * MT * TPW * 1024;
     static_assert(stage + reduce <= kMaxLds, "the two staged steps and the reduction fit a block's LDS");
-    const bool few = M <= 8 && !CM;
+    const bool few = M <= 8 && !CM && OUT != kOutPairSilu; /* the pair ends in BF16 */
     const int period = few ? kFoldFew : kFold;
-    const bool fold = K / 128 > (few ? kFoldFew : WK == 2 ? kFoldFromTwo : kFoldFrom) * WK;
+    const bool fold = K / 128 > (few ? kFoldFewFrom : WK == 2 ? kFoldFromTwo : kFoldFrom) * WK;
     const size_t smem = fold ? stage + reduce : std::max(stage, reduce);
     constexpr size_t elem = OUT == kOutF32 ? 4 : 2;
     const int cols = (((N / 8 + 1) / 2 + WN * TPW - 1) / (WN * TPW) + 7) / 8 * 8;
@@ -2579,7 +2579,7 @@ int launch_rows_stream(const uint16_t *x, int M, const uint8_t *w, const uint16_
     const size_t smem = std::max(((size_t)(K / 128) * M * 256 + 1023) / 1024 * 1024, (size_t)32 * 1024);
     if (M > 16 || TPB > 16 || smem > kMaxLds) return 1;
     /* a wave has TPB G / 16 units, of one tile pair at most G */
-    const bool fold = std::min(K / 128, (TPB * (K / 128) + 15) / 16) > (CM ? kFoldFrom : kFoldFew);
+    const bool fold = std::min(K / 128, (TPB * (K / 128) + 15) / 16) > (CM ? kFoldFrom : kFoldFewFrom);
     launch_k((fold ? rows_stream_kernel<OUT_F32, CM, true> : rows_stream_kernel<OUT_F32, CM, false>),
              dim3((tile_pairs + TPB - 1) / TPB), dim3(1024), smem, stream, x, M, w, s, out, N, K, TPB, residual);
     return hip_status(hipGetLastError(), "rows stream launch");

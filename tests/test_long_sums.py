@@ -16,6 +16,7 @@ BOUNDS = [
                    (128, 2, 1.6784e-7), (200, 1, 1.6701e-7)]),
     (4096, 12288, [(33, 2, 1.6376e-7), (128, 2, 1.6341e-7), (200, 1, 1.6379e-7)]),
     (4096, 10240, [(33, 2, 1.6190e-7), (128, 2, 1.6351e-7), (200, 1, 1.6134e-7)]),
+    (5120, 8064, [(5, 20, 1.5409e-7), (8, 20, 1.5636e-7)]),
     (5120, 8704, [(17, 4, 1.6370e-7), (64, 2, 1.6362e-7), (200, 1, 1.6335e-7)]),
     (5120, 5120, [(64, 2, 1.6175e-7), (200, 2, 1.6275e-7)]),
     (16384, 16384, [(2, 10, 1.6763e-7), (4, 10, 1.7397e-7)]),
