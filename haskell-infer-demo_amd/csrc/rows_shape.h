@@ -60,8 +60,8 @@ inline std::size_t rows_smem(int M, int K, int waves) {
 
 /* Whether an N x K linear of M <= 16 row-major rows that no LDS-staged tile-pair kernel takes runs on
  * rows_stream_kernel (or past its LDS on the row-tiled GEMM): with more than one tile pair a CU, from a K that falls
- * with the rows (17408 x 5120 M = 2 / 3 / 8 18.8 / 19.6 / 30.8 us in the few-row form, 17.1 / 17.2 / 21.3 there;
- * 8704 x 5120 M = 5 / 8 12.1 / 12.6, 10.3 / 10.8). With up to two tile pairs a CU the few-row form keeps 4 rows a
+ * with the rows (17408 x 5120 M = 2 / 3 / 8 18.9 / 19.4 / 31.1 us in the few-row form, 17.6 / 17.1 / 21.5 there;
+ * 8704 x 5120 M = 5 / 8 11.9 / 12.6, 10.2 / 10.8). With up to two tile pairs a CU the few-row form keeps 4 rows a
  * little longer (8704 x 5120 10.4 / 10.4) and up to 64 KB of rows (5 rows of 5248 x 4224 7.3 / 7.8, of 6144 x 8192
  * 9.2 / 9.5, but 6 of 6144 x 5120 8.4 / 8.2, and 5 of 5248 x 9728 11.5 / 10.0); and just past one tile pair a CU, where
  * the streamed kernel leaves half of the CUs without a block, as long as two blocks of it fit a CU (5 rows of
